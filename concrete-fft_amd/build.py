@@ -28,7 +28,8 @@ HIP_FLAGS = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang",
              "-packed-fp32-ops", "-munsafe-fp-atomics"]
 
 HIP_SOURCES = ["fft_kernels.hip", "polymul_kernels.hip", "polymul_n2048_kernels.hip", "fft128_kernels.hip",
-               "exact_kernels.hip", "extprod_kernels.hip", "uneven_kernels.hip", "noalloc.hip", "serve_kernels.hip",
+               "exact_kernels.hip", "extprod_kernels.hip",
+               "extprod_fused_kernels.hip", "uneven_kernels.hip", "noalloc.hip", "serve_kernels.hip",
                "large_transform_kernels.hip", "dit16_kernels.hip", "fixed_n256.hip", "fixed_n512.hip",
                "fixed_n1024.hip", "fixed_n2048.hip", "fixed_n4096.hip",
                "fixed_n8192.hip"]

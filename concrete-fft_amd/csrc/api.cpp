@@ -236,6 +236,11 @@ int build_f64_plan(cfft_plan_s *p) {
   if (p->kind == cfft_plan_s::UNORDERED) {
     const size_t N = 2 * n;
     std::vector<cfft_host::C64> tws = cfft_host::twist_table(N), utw = cfft_host::untwist_table(N);
+    p->twist_mirrored = true;
+    for (size_t j = 1; j < n / 2 && p->twist_mirrored; ++j) {
+      const cfft_host::C64 m{tws[j].im, tws[j].re};
+      p->twist_mirrored = std::memcmp(&m, &tws[n - j], sizeof m) == 0;
+    }
     CFFT_HIP(hipMalloc(&p->d_twist, n * sizeof(dc64)));
     CFFT_HIP(hipMalloc(&p->d_untwist, n * sizeof(dc64)));
     CFFT_HIP(hipMemcpy(p->d_twist, tws.data(), n * sizeof(dc64), hipMemcpyHostToDevice));

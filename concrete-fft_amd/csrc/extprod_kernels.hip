@@ -11,10 +11,9 @@
 // (level 0 most significant).
 #include <hip/hip_runtime.h>
 
-#include "lds_attr.hpp"
-
-
+#include "gadget.hpp"
 #include "launch.hpp"
+#include "lds_attr.hpp"
 #include "r16_exec.hpp"
 #include "stockham_exec.hpp"
 
@@ -23,40 +22,6 @@ using cfft_launch::dc64;
 using cfft_prog::Program;
 
 namespace {
-
-// One level of the gadget decomposition, without branches or loops: the
-// balanced digits of the rounded value st (rep = levels * base_log bits) are
-// the plain base-2^B digits of st + (half in every digit position), each
-// minus half -- the carry loop of the decomposition done by one addition
-// (the same digits; the wrap-around past rep bits is the top digit's carry,
-// which the decomposition drops as well).
-struct Gadget {
-  uint32_t shift;   // 64 - rep: the rounding position (0: no rounding)
-  uint32_t down;    // base_log * (levels - 1 - level): this level's digit position
-  uint64_t keep;    // the low rep bits
-  uint64_t offset;  // half in every digit position
-  uint64_t mask;    // one digit
-  int64_t half;
-};
-
-__device__ __forceinline__ Gadget gadget_of(uint32_t level, uint32_t levels, uint32_t base_log) {
-  Gadget g;
-  const uint32_t rep = levels * base_log;
-  g.shift = 64 - rep;
-  g.down = base_log * (levels - 1 - level);
-  g.keep = rep < 64 ? ((uint64_t)1 << rep) - 1 : ~(uint64_t)0;
-  g.mask = ((uint64_t)1 << base_log) - 1;
-  g.half = (int64_t)1 << (base_log - 1);
-  g.offset = 0;
-  for (uint32_t i = 0; i < levels; ++i) g.offset = (g.offset << base_log) | (uint64_t)g.half;
-  return g;
-}
-
-__device__ __forceinline__ int64_t gadget_digit(const Gadget &g, uint64_t x) {
-  const uint64_t up = g.shift ? (x >> (g.shift - 1)) & 1u : 0;  // ties round up
-  const uint64_t st = ((x >> g.shift) + up) & g.keep;
-  return (int64_t)(((st + g.offset) >> g.down) & g.mask) - g.half;
-}
 
 // key: npolys u64 torus polynomials -> Fourier (plan order), one per transform
 template <int E>

@@ -51,6 +51,9 @@ struct cfft_plan_s {
   cfft_launch::dc64 *d_tw_r8 = nullptr;
   // negacyclic product tables (N = 2n)
   cfft_launch::dc64 *d_twist = nullptr, *d_untwist = nullptr;
+  // d_twist[n - j] is d_twist[j] with re and im exchanged, bit for bit, for
+  // every 0 < j < n/2 (kernels that stage half of the table rely on it)
+  bool twist_mirrored = false;
 
   // fft128
   double *d_tw128 = nullptr;  // 4 x n: re0 | re1 | im0 | im1

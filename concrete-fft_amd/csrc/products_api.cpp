@@ -37,14 +37,21 @@ hipError_t external_product_split_w(uint32_t log2n, const dc64 *keyf, const uint
                                     uint32_t levels, uint32_t base_log, const dc64 *tw,
                                     const dc64 *tw_blk, const dc64 *twist, const dc64 *untwist,
                                     dc64 *scratch, hipStream_t s);
+bool external_product_fused_supported(uint32_t log2n, uint64_t batch, uint32_t k1,
+                                      uint32_t levels);
+hipError_t external_product_fused(uint32_t log2n, const dc64 *keyf, const uint64_t *glwe,
+                                  const uint64_t *glwe_tab, uint64_t *out,
+                                  const uint64_t *out_tab, uint64_t batch, uint32_t k1,
+                                  uint32_t levels, uint32_t base_log, const dc64 *tw,
+                                  const dc64 *tw_blk, const dc64 *twist, hipStream_t s);
 }
 
 namespace {
-// The external product runs split (rows and columns over workgroups through a
-// Fourier scratch) at every batch size: measured faster than one workgroup
-// per GLWE from batch 1 to 4096 at N = 1024, 2048 and 4096.  Large batches
-// run in passes over one scratch of at most kSplitMaxRows spectra and
-// kSplitMaxBytes, a whole number of GLWEs per pass.
+// The split form of the external product (rows and columns over workgroups
+// through a Fourier scratch): for plans and shapes the one-launch form does
+// not take, and buffers that overlap.  Large batches run in passes over one
+// scratch of at most kSplitMaxRows spectra and kSplitMaxBytes, a whole number
+// of GLWEs per pass.
 constexpr uint64_t kSplitMaxRows = 16384;
 constexpr uint64_t kSplitMaxBytes = (uint64_t)256 << 20;
 constexpr int kMaxK1 = 64;
@@ -111,9 +118,6 @@ int external_product_with_scratch(cfft_plan plan, const void *key_fourier, int k
   if ((glwe_tab || out_tab) && !external_product_tables_supported(plan))
     return set_error(CFFT_ERROR_WRONG_PLAN_KIND,
                      "address tables need the wave-local split kernels (Dif16, N = 1024 ... 4096)");
-  // Rows (digit polynomials) and columns spread over workgroups through a
-  // Fourier scratch: measured faster than one workgroup per GLWE from batch 1
-  // to 4096 at N = 1024, 2048 and 4096.
   hipError_t e = hipSuccess;
   uint64_t per_pass = glwe_per_pass(plan, k1, levels);
   size_t bytes = external_product_scratch_bytes(plan, k1, levels, batch);
@@ -129,6 +133,21 @@ int external_product_with_scratch(cfft_plan plan, const void *key_fourier, int k
     bytes = 0;
   }
   hipStream_t s = stream;
+  const cfft_launch::dc64 *blk = split_w_block(plan);
+  const size_t glwe_words = (size_t)k1 * 2 * plan->n;  // one GLWE: k1 polynomials of N words
+  // One launch, no scratch.  It writes a GLWE's result while later GLWEs are
+  // still to be read, so buffers that overlap other than exactly keep the
+  // split form, which reads a whole pass before it writes.
+  const size_t span = batch * glwe_words;
+  const bool shifted = glwe && out && glwe != out && glwe < out + span && out < glwe + span;
+  if (blk && !shifted && (plan->n < 2048 || plan->twist_mirrored) &&
+      cfft_launch::external_product_fused_supported(ilog2(plan->n), batch, (uint32_t)k1,
+                                                    (uint32_t)levels))
+    return hip_error(cfft_launch::external_product_fused(
+                         ilog2(plan->n), reinterpret_cast<const cfft_launch::dc64 *>(key_fourier),
+                         glwe, glwe_tab, out, out_tab, batch, (uint32_t)k1, (uint32_t)levels,
+                         (uint32_t)base_log, plan->d_tw, blk, plan->d_twist, s),
+                     "external product (fused)");
   // the caller's scratch when it holds one pass's spectra, else the cache
   cfft_internal::ScratchLease lease;
   if (!no_alloc && (!scratch || scratch_bytes < bytes)) {
@@ -136,7 +155,6 @@ int external_product_with_scratch(cfft_plan plan, const void *key_fourier, int k
     if (e != hipSuccess) return hip_error(e, "external product scratch");
   }
   cfft_launch::dc64 *S = reinterpret_cast<cfft_launch::dc64 *>(lease.ptr ? lease.ptr : scratch);
-  const size_t glwe_words = (size_t)k1 * 2 * plan->n;  // one GLWE: k1 polynomials of N words
   for (uint64_t off = 0; off < batch && e == hipSuccess; off += per_pass) {
     const uint64_t m = batch - off < per_pass ? batch - off : per_pass;
     const uint64_t *g = glwe ? glwe + off * glwe_words : nullptr;
@@ -148,7 +166,6 @@ int external_product_with_scratch(cfft_plan plan, const void *key_fourier, int k
     // at n = 512).  Measured at N = 4096 against two waves per row transform
     // in the generic split form: 45 vs 72 us for 16 GLWEs, 155 vs 402 us for
     // 1024, 0.86 vs 1.52 ms for 4096.
-    const cfft_launch::dc64 *blk = split_w_block(plan);
     if (blk)
       e = cfft_launch::external_product_split_w(
           ilog2(plan->n), reinterpret_cast<const cfft_launch::dc64 *>(key_fourier), g, gt, o, ot,

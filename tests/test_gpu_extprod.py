@@ -143,3 +143,36 @@ def test_large_batch_runs_in_passes(cfft, oracle):
     for b in (0, 1023, 1024, 1099):
         assert np.array_equal(whole[b], oracle.external_product(N, k1, levels, base_log, kfh, 6,
                                                                 512, glwe[b])), b
+
+
+@pytest.mark.parametrize("N,k1,levels,base_log,batch", [
+    (1024, 2, 3, 8, 1), (1024, 3, 2, 10, 257), (1024, 2, 1, 23, 1029), (1024, 4, 5, 6, 515),
+    (2048, 2, 3, 8, 1), (2048, 4, 5, 6, 258), (2048, 2, 3, 8, 1027), (2048, 3, 2, 16, 513),
+    (4096, 2, 2, 15, 1), (4096, 3, 1, 23, 259), (4096, 2, 3, 8, 515), (4096, 4, 3, 8, 2),
+])
+def test_fused_product_groups(cfft, oracle, N, k1, levels, base_log, batch):
+    """The one-launch form (k1 = 2 ... 4): 1, 2 or 4 GLWEs per workgroup
+    (up to 256, 512 and more GLWEs), a last group only partly filled, a
+    second group per workgroup, rows filling one round, several or part of
+    one; in place gives the same words, and so does an output shifted by one
+    GLWE over the input (the split form)."""
+    from cfft_amd import lib, check
+    from cfft_amd.device import DeviceBuffer
+    print("fused product: N=%d k1=%d levels=%d batch=%d" % (N, k1, levels, batch), flush=True)
+    base_n = min(N // 2, 1024)
+    rng = np.random.default_rng(N + 10 * k1 + levels + batch)
+    key = rng.integers(0, M, (k1 * levels, k1, N), dtype=np.uint64)
+    glwe = rng.integers(0, M, (batch, k1, N), dtype=np.uint64)
+    plan = _plan(N, 6, base_n)
+    kf = _key_fourier(plan, key, k1, levels)
+    got = _extprod(plan, kf, k1, levels, base_log, glwe)
+    kfh = oracle.torus_to_fourier(key, 6, base_n)
+    for b in sorted({0, 1 % batch, batch // 2, max(0, batch - 2), batch - 1}):
+        want = oracle.external_product(N, k1, levels, base_log, kfh, 6, base_n, glwe[b])
+        assert np.array_equal(got[b], want), (b, int(np.sum(got[b] != want)))
+    both = np.concatenate([glwe, np.zeros((1, k1, N), np.uint64)])
+    for shift in (0, 1):
+        d = DeviceBuffer.from_host(both)
+        check(lib.cfft_external_product(plan.handle, kf.dptr, k1, levels, base_log, d.dptr,
+                                        d.dptr + shift * k1 * N * 8, batch, None))
+        assert np.array_equal(d.download()[shift:batch + shift], got), shift
