@@ -25,7 +25,7 @@
 // against the split form (two launches, spectra through HBM), us per call,
 // k1 = 2, l = 3: N = 1024 18.7 -> 10.2 (1 GLWE), 31.6 -> 11.7 (256), 75.5 ->
 // 40.0 (2000); N = 2048 19.9 -> 13.1, 37.8 -> 15.3, 127 -> 71; N = 4096 34.2
-// -> 25.7, 55.0 -> 30.1, 287 -> 190.
+// -> 24.1, 54.6 -> 28.6, 285 -> 167.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -300,7 +300,7 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
       auto fetch_next = [&]() {
         fetch(more ? g0 : g0 + (uint64_t)gridDim.x * P, more ? r0 + RG : 0);
       };
-      if constexpr (CH == 1) fetch_next();
+      if constexpr (CH == 1 || NARROW) fetch_next();
       sched_fence();
       __syncthreads();
       const uint32_t t = launder_u32(tid);
@@ -323,9 +323,9 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
           }
         }
       }
-      if constexpr (CH == 2) {
+      if constexpr (CH == 2 && !NARROW) {
         sched_fence();
-        fetch_next();  // (beside the key points it would spill)
+        fetch_next();  // (64-bit words would spill beside the key points)
       }
       __syncthreads();  // every spectrum of the round read
     }
@@ -352,16 +352,6 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
       for (uint32_t m = 0; m < 16; ++m) v[m] = x[l + T * m];
       base_transform<F::LB, false>(v, x, l, ltw);
     }
-    if (CH == 2 && busy && ch == 1) {
-      // DEPTH_INV radix 2: conj(T[q]) on chunk 1's point before the butterfly
-      const c64 *tj = launder(tw);
-#pragma unroll
-      for (uint32_t s0 = 0; s0 < 16; s0 += 8) {
-#pragma unroll
-        for (uint32_t s = s0; s < s0 + 8; ++s) v[s] = cmul(conj(tj[l + 64 * S::end_m(s)]), v[s]);
-        sched_fence();
-      }
-    }
     // untwist = conj(twist) / n (an exact scaling: the plan's untwist table)
     auto put = [&](uint64_t *o, uint32_t c2, uint32_t i, c64 y) {
       const c64 z = twist_point<CH>(ltz, c2, i);
@@ -387,6 +377,7 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
     for (uint32_t e = 0; e < F::PB; ++e) {
       const uint32_t idx = t + 64 * kFWaves * e;
       const uint32_t q = (idx & (T - 1)) + T * S::end_m(idx / T);
+      const c64 zq = CH == 2 ? tw[q] : mk(0.0, 0.0);
 #pragma unroll
       for (int g = 0; g < P; ++g) {
         if (g0 + g >= batch) break;
@@ -397,8 +388,10 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
           if constexpr (CH == 1) {
             put(o, 0, q, y[0]);
           } else {
-            put(o, 0, q, cadd(y[0], y[F::nb]));
-            put(o, 1, q, csub(y[0], y[F::nb]));
+            // DEPTH_INV radix 2: conj(T[q]) on chunk 1's point, then the butterfly
+            const c64 b = cmul(conj(zq), y[F::nb]);
+            put(o, 0, q, cadd(y[0], b));
+            put(o, 1, q, csub(y[0], b));
           }
         }
       }
@@ -475,14 +468,19 @@ hipError_t launch_fused_k(const FArgs &a, uint32_t k1, hipStream_t s) {
 namespace cfft_launch {
 
 // The one-launch form takes k1 = 2 ... 4 (its column sums are registers).  It
-// measured faster than the split form over N = 1024, 2048, 4096, 2 to 16 rows
-// and 1 to 2000 GLWEs (1.1x to 2.7x), except at N = 4096 with 16 rows and few
-// GLWEs, where one CU runs in four rounds the rows that the split form spreads
-// over idle CUs: 52.5 against 46.4 us for one GLWE, 55.8 against 66.3 for 64.
+// measured 1.1x to 2.7x faster than the split form over N = 1024, 2048, 4096,
+// 2 to 12 rows and 1 to 2000 GLWEs.  With many rows and few GLWEs one CU runs
+// in rounds the rows that the split form spreads over idle CUs: from 4 rounds
+// on the split form is ahead below about 2 rounds^2 GLWEs (us, split against
+// fused: N = 4096, 16 rows, 4 rounds: 51.9 / 60.2 for 8 GLWEs, 64.0 / 61.1 for
+// 40; 32 rows, 8 rounds: 100 / 126 for 64, 288 / 251 for 260; N = 2048, 32
+// rows: 52.0 / 56.8 for 24, 57.7 / 57.0 for 40).
 bool external_product_fused_supported(uint32_t log2n, uint64_t batch, uint32_t k1,
                                       uint32_t levels) {
-  if (log2n == 11 && batch < 64 && k1 * levels >= 16) return false;
-  return log2n >= 9 && log2n <= 11 && k1 >= 2 && k1 <= 4;
+  if (log2n < 9 || log2n > 11 || k1 < 2 || k1 > 4) return false;
+  const uint32_t rows_per_round = log2n == 9 ? 16 : log2n == 10 ? 8 : 4;
+  const uint64_t rounds = (k1 * levels + rows_per_round - 1) / rows_per_round;
+  return rounds < 4 || batch >= 2 * rounds * rounds;
 }
 
 hipError_t external_product_fused(uint32_t log2n, const dc64 *keyf, const uint64_t *glwe,
