@@ -16,6 +16,7 @@
 #include "cfft.h"
 #include "host_tables.hpp"
 #include "launch.hpp"
+#include "lds_attr.hpp"
 #include "plan.hpp"
 #include "host_stage.hpp"
 #include "scratch.hpp"
@@ -149,8 +150,12 @@ int build_f64_plan(cfft_plan_s *p) {
 
   // tables
   std::vector<cfft_host::C64> tw = cfft_host::twiddle_table(n);
-  CFFT_HIP(hipMalloc(&p->d_tw, n * sizeof(dc64)));
-  CFFT_HIP(hipMemcpy(p->d_tw, tw.data(), n * sizeof(dc64), hipMemcpyHostToDevice));
+  // the n-point table, then the base transform's own entries T[j n / base_n]
+  const size_t base_tw = p->base_n < n ? p->base_n : 0;
+  std::vector<cfft_host::C64> tw_all(tw);
+  for (size_t j = 0; j < base_tw; ++j) tw_all.push_back(tw[j * (n / p->base_n)]);
+  CFFT_HIP(hipMalloc(&p->d_tw, tw_all.size() * sizeof(dc64)));
+  CFFT_HIP(hipMemcpy(p->d_tw, tw_all.data(), tw_all.size() * sizeof(dc64), hipMemcpyHostToDevice));
   const bool dit16 = p->algo == CFFT_DIT16 && p->base_n == n && n == 1024;
   if ((p->algo == CFFT_DIF16 && p->base_n == n && cfft_launch::r16_supported(log2n)) || dit16) {
     const size_t T = n / 16, T2 = T / 16;
@@ -904,6 +909,25 @@ int cfft_negacyclic_polymul_u64(cfft_plan plan, const uint64_t *a, const int64_t
 int cfft_polymul_dispatch(const cfft_plan_s *p, const uint64_t *a, const int64_t *b, uint64_t *c,
                           size_t batch, hipStream_t s) {
   const uint32_t log2n = ilog2(p->n);
+  auto program = [&] {
+    return hip_error(cfft_launch::polymul_generic(p->fwd_full, p->inv_full, a, b, c, batch, p->d_tw,
+                                                  p->d_twist, p->d_untwist, s),
+                     "polymul");
+  };
+  // Dif16 at up to 8192 coefficients per CU: the register-resident kernels
+  // below give a product one wave (or, above N = 2048, a workgroup of eight)
+  // and stage tables for every workgroup, which pays once the batch fills them
+  // several times; until then the eight-point schedule's n / 8 threads per
+  // product finish earlier.  us, this against them: N = 1024 7.2 / 8.6 (1
+  // product), 15.4 / 19.3 (2048), 27.3 / 23.3 (4096); N = 2048 8.3 / 9.5, 16.1 /
+  // 19.1 (1024), 28.3 / 22.6 (2048); N = 4096 11.6 / 22.2, 19.5 / 26.4 (512),
+  // 32.5 / 29.3 (1024); N = 8192 18.4 / 21.4, 23.3 / 26.1 (256), 39.9 / 30.4
+  // (512); N = 2048 on base 512 8.4 / 11.2, 17.1 / 24.1 (1024), 29.4 / 27.5.
+  if (p->algo == CFFT_DIF16 && p->n >= 512 && p->n <= 4096 && p->base_n >= 512) {
+    int cus = 0;
+    CFFT_HIP(cfft_launch::cu_count(&cus));
+    if (batch <= (size_t)cus * 8192 / (2 * p->n)) return program();
+  }
   if ((p->n == 256 || p->n == 512) && p->base_n == p->n && p->d_tw_base1024)  // Dif16
     return hip_error(cfft_launch::wsub_polymul(log2n, a, b, c, batch, p->d_tw_base1024,
                                                p->d_twist, s),
@@ -926,7 +950,5 @@ int cfft_polymul_dispatch(const cfft_plan_s *p, const uint64_t *a, const int64_t
     return hip_error(cfft_launch::wd2_512_polymul(a, b, c, batch, p->d_tw, p->d_tw_base1024,
                                                   p->d_twist, s),
                      "wd2_512_polymul");
-  return hip_error(cfft_launch::polymul_generic(p->fwd_full, p->inv_full, a, b, c, batch, p->d_tw,
-                                                p->d_twist, p->d_untwist, s),
-                   "polymul");
+  return program();
 }

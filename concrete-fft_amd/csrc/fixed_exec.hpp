@@ -57,7 +57,8 @@ using cfft_prog::Program;
 
 // The generic fused product (k_polymul_generic) for one (algo, n, base_n)
 // fixed at compile time: the forward and inverse programs are
-// cfft_prog::fixed_program's, unrolled with constant pass fields.
+// cfft_prog::fixed_program's, unrolled with constant pass fields.  (Dit16
+// products; the other algos run fixed8_polymul.hpp.)
 template <int ALGO, int LOG2N, int LOG2BN, bool FWD>
 struct FixedProg {
   static constexpr Program prog = cfft_prog::fixed_program(ALGO, LOG2N, LOG2BN, FWD);

@@ -1,6 +1,8 @@
-// fixed_n1024.hip -- compile-time pass programs (fixed_exec.hpp) for n = 1024:
-// every algo on bases 1024 and 512 except those with a register-resident kernel
-// (Dif16 / 1024, Dit16 / 1024, Dif8 / 1024, Dif16 / 512).
+// fixed_n1024.hip -- compile-time pass programs (products: fixed8_polymul.hpp,
+// Dit16 and transforms: fixed_exec.hpp) for n = 1024: every algo on bases 1024
+// and 512 except those with a register-resident kernel (Dit16 / 1024 and Dif8 /
+// 1024; Dif16 for its transforms and large product batches).
+#include "fixed8_polymul.hpp"
 #include "fixed_exec.hpp"
 
 namespace cfft_launch {
@@ -12,17 +14,19 @@ bool fixed_polymul_n1024(const cfft_prog::Program &fwd, const cfft_prog::Program
   const c64 *t = reinterpret_cast<const c64 *>(tw);
   const c64 *tws = reinterpret_cast<const c64 *>(twist);
   const c64 *utw = reinterpret_cast<const c64 *>(untwist);
-  return fixed_polymul_try<0, 10, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<1, 10, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<2, 10, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<3, 10, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<5, 10, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<0, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<1, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<2, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<3, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<4, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<5, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+  return fixed8_polymul_try<6, 10, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<6, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<0, 10, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<1, 10, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<2, 10, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<3, 10, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<5, 10, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<0, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<1, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<2, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<3, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<4, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<5, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
          fixed_polymul_try<7, 10, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e);
 }
 

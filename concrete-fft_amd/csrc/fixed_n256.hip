@@ -1,6 +1,7 @@
-// fixed_n256.hip -- compile-time pass programs (fixed_exec.hpp) for n = 256:
-// every algo on base 256 (the autotuner's base for n = 256) except Dif16
-// (register-resident).
+// fixed_n256.hip -- compile-time pass programs (products: fixed8_polymul.hpp,
+// Dit16 and transforms: fixed_exec.hpp) for n = 256: every algo on base 256 (the
+// autotuner's base for n = 256) except Dif16 (register-resident).
+#include "fixed8_polymul.hpp"
 #include "fixed_exec.hpp"
 
 namespace cfft_launch {
@@ -12,12 +13,12 @@ bool fixed_polymul_n256(const cfft_prog::Program &fwd, const cfft_prog::Program 
   const c64 *t = reinterpret_cast<const c64 *>(tw);
   const c64 *tws = reinterpret_cast<const c64 *>(twist);
   const c64 *utw = reinterpret_cast<const c64 *>(untwist);
-  return fixed_polymul_try<0, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<1, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<2, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<3, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<4, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<5, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+  return fixed8_polymul_try<0, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<1, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<2, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<3, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<4, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<5, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
          fixed_polymul_try<7, 8, 8>(fwd, inv, a, b, c, batch, t, tws, utw, s, e);
 }
 

@@ -1,6 +1,8 @@
-// fixed_n4096.hip -- compile-time pass programs (fixed_exec.hpp) for n = 4096:
-// every algo on bases 1024 and 512 (and, for the transforms, the ordered
-// plans' base_n = n) except Dif16 / 1024 (register-resident).
+// fixed_n4096.hip -- compile-time pass programs (products: fixed8_polymul.hpp,
+// Dit16 and transforms: fixed_exec.hpp) for n = 4096: every algo on bases 1024 and
+// 512 (and, for the transforms, the ordered plans' base_n = n); Dif16 / 1024 for
+// small product batches (else register-resident).
+#include "fixed8_polymul.hpp"
 #include "fixed_exec.hpp"
 
 namespace cfft_launch {
@@ -12,20 +14,21 @@ bool fixed_polymul_n4096(const cfft_prog::Program &fwd, const cfft_prog::Program
   const c64 *t = reinterpret_cast<const c64 *>(tw);
   const c64 *tws = reinterpret_cast<const c64 *>(twist);
   const c64 *utw = reinterpret_cast<const c64 *>(untwist);
-  return fixed_polymul_try<0, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<1, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<2, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<3, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<4, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<5, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+  return fixed8_polymul_try<6, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<0, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<1, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<2, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<3, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<4, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<5, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
          fixed_polymul_try<7, 12, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<0, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<1, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<2, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<3, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<4, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<5, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<6, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<0, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<1, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<2, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<3, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<4, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<5, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<6, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
          fixed_polymul_try<7, 12, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e);
 }
 

@@ -1,5 +1,8 @@
-// fixed_n512.hip -- compile-time pass programs (fixed_exec.hpp) for n = 512:
-// every algo on base 512 except Dif16 (register-resident).
+// fixed_n512.hip -- compile-time pass programs (products: fixed8_polymul.hpp,
+// Dit16 and transforms: fixed_exec.hpp) for n = 512: every algo on base 512
+// (Dif16 for small product batches; its transforms and large ones are
+// register-resident).
+#include "fixed8_polymul.hpp"
 #include "fixed_exec.hpp"
 
 namespace cfft_launch {
@@ -11,12 +14,13 @@ bool fixed_polymul_n512(const cfft_prog::Program &fwd, const cfft_prog::Program 
   const c64 *t = reinterpret_cast<const c64 *>(tw);
   const c64 *tws = reinterpret_cast<const c64 *>(twist);
   const c64 *utw = reinterpret_cast<const c64 *>(untwist);
-  return fixed_polymul_try<0, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<1, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<2, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<3, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<4, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<5, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+  return fixed8_polymul_try<6, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<0, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<1, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<2, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<3, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<4, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<5, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
          fixed_polymul_try<7, 9, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e);
 }
 

@@ -1,5 +1,7 @@
-// fixed_n8192.hip -- compile-time pass programs (fixed_exec.hpp) for n = 8192:
-// every algo on bases 1024 and 512 except Dif16 / 1024 (register-resident).
+// fixed_n8192.hip -- compile-time pass programs (products: fixed8_polymul.hpp,
+// Dit16 and transforms: fixed_exec.hpp) for n = 8192: every algo on bases 1024
+// and 512 except Dif16 / 1024 (register-resident).
+#include "fixed8_polymul.hpp"
 #include "fixed_exec.hpp"
 
 namespace cfft_launch {
@@ -11,20 +13,20 @@ bool fixed_polymul_n8192(const cfft_prog::Program &fwd, const cfft_prog::Program
   const c64 *t = reinterpret_cast<const c64 *>(tw);
   const c64 *tws = reinterpret_cast<const c64 *>(twist);
   const c64 *utw = reinterpret_cast<const c64 *>(untwist);
-  return fixed_polymul_try<0, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<1, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<2, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<3, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<4, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<5, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+  return fixed8_polymul_try<0, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<1, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<2, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<3, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<4, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<5, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
          fixed_polymul_try<7, 13, 10>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<0, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<1, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<2, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<3, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<4, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<5, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
-         fixed_polymul_try<6, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<0, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<1, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<2, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<3, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<4, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<5, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
+         fixed8_polymul_try<6, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e) ||
          fixed_polymul_try<7, 13, 9>(fwd, inv, a, b, c, batch, t, tws, utw, s, e);
 }
 

@@ -20,7 +20,9 @@ struct cfft_plan_s {
   int device = 0;
 
   // f64 path
-  cfft_launch::dc64 *d_tw = nullptr;  // T[j] = (cos, sin)(-2 pi j / n)
+  // T[j] = (cos, sin)(-2 pi j / n), j < n; with base_n < n then T[j n / base_n],
+  // j < base_n
+  cfft_launch::dc64 *d_tw = nullptr;
   uint32_t *d_freq = nullptr;         // position -> frequency
   uint32_t *d_pos = nullptr;          // frequency -> position
   std::vector<uint32_t> pos_of_freq;  // host copy of d_pos

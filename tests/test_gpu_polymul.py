@@ -219,3 +219,45 @@ def test_depth_product_rounds(cfft, oracle, N, batch):
     c = products.negacyclic_polymul_u64_host(plan, a, b)
     ref = oracle.polymul_f64(a, b, 6, 1024, threads=16)
     assert np.array_equal(c, ref), (N, batch, int(np.sum(c != ref)))
+
+
+EIGHT_POINT = [(512, algo, 256) for algo in range(6)] + [
+    (N, algo, base_n) for N in (1024, 2048, 4096, 8192, 16384) for algo in range(7)
+    for base_n in (512, 1024) if 2 * base_n <= N and (N, algo, base_n) not in
+    ((2048, 4, 1024), (16384, 6, 1024))]
+
+
+@pytest.mark.parametrize("N,algo,base_n", EIGHT_POINT)
+def test_eight_point_products(cfft, oracle, N, algo, base_n):
+    """The compile-time programs on eight points per thread, every plan that
+    runs on them: one product, and 3 (at N = 512 two products share a
+    workgroup, so the last is half empty), extreme operands included,
+    bit-exact against the oracle."""
+    from cfft_amd import products
+    from cfft_amd.unordered import FftAlgo, Method, Plan
+    print("eight-point product: N=%d algo=%d base_n=%d" % (N, algo, base_n), flush=True)
+    plan = Plan(N // 2, Method.UserProvided(FftAlgo(algo), base_n))
+    a, b = rand_inputs(N + 17 * algo, 3, N)
+    a[1, :5] = [0, 2**64 - 1, 1 << 63, (1 << 63) - 1, 1]
+    b[1, :] = np.where(np.arange(N) % 2, -128, 127)
+    ref = oracle.polymul_f64(a, b, algo, base_n)
+    for batch in (1, 3):
+        c = products.negacyclic_polymul_u64_host(plan, a[3 - batch:], b[3 - batch:])
+        assert np.array_equal(c, ref[3 - batch:]), batch
+
+
+@pytest.mark.parametrize("N,base_n", [(1024, 512), (2048, 512), (2048, 1024), (4096, 1024),
+                                      (8192, 1024)])
+def test_dif16_product_routes_meet(cfft, oracle, N, base_n):
+    """Dif16 products change kernels at 8192 coefficients per CU: the largest
+    batch of the eight-point kernel and the smallest of the register-resident
+    one give the oracle's words."""
+    from cfft_amd import products
+    from cfft_amd.unordered import FftAlgo, Method, Plan
+    plan = Plan(N // 2, Method.UserProvided(FftAlgo.Dif16, base_n))
+    last = 256 * 8192 // N
+    a, b = rand_inputs(N + base_n, last + 1, N)
+    ref = oracle.polymul_f64(a, b, 6, base_n)
+    for batch in (last, last + 1):
+        c = products.negacyclic_polymul_u64_host(plan, a[:batch], b[:batch])
+        assert np.array_equal(c, ref[:batch]), batch
