@@ -20,8 +20,9 @@ constexpr size_t kLdsBytes = kLdsPoints * 16;
 // base_n < 1024 at column stride 1024 / base_n)
 constexpr uint32_t kTwR16Points = 16 * 64 + 16 * 4;
 constexpr size_t kR16LdsBytes = (size_t)(kLdsPoints + kTwR16Points) * 16;
-// device work queue of the Dif16 body: partitions (one counter each, on its
-// own 128-byte line) and the counter buffer's layout
+// device work queue of the Dif16 body: partitions (two words each, next index
+// and workgroups done, on a 128-byte line of its own; zero between launches)
+// and the counter buffer's layout
 constexpr uint32_t kQueueParts = 8;
 constexpr uint32_t kCounterStride = 32;  // words
 constexpr uint32_t kGenericCounter = kQueueParts * kCounterStride;
@@ -75,15 +76,15 @@ constexpr uint32_t jobs_per_tile(uint32_t log2n, bool r16) {
 
 // sets the kernels' LDS limit on the current device (before any launch)
 hipError_t prepare();
-// Generic body: resets counter[0], then runs tiles[0 .. ntiles) on `grid`
-// persistent workgroups.
+// Generic body: runs tiles[0 .. ntiles) on `grid` persistent workgroups, fed by
+// the queue at counter[0 .. 1].
 hipError_t launch_persistent(const UJob *jobs, const uint32_t *order, const UTile *tiles,
                              uint32_t ntiles, const UClass *classes, uint32_t *counter,
                              uint32_t grid, const double *in, cfft_launch::dc64 *fourier,
                              double *out, hipStream_t s);
 // Dif16 body: runs tiles[0 .. ntiles) on `grid` persistent workgroups, fed
-// by the partitioned device queue at `counter` (kQueueParts counters, reset
-// by a kernel launched first) or, with counter null, dealt round-robin.
+// by the partitioned device queue at `counter` (kQueueParts queues) or, with
+// counter null, dealt round-robin.
 hipError_t launch_r16_persistent(const UJob *jobs, const uint32_t *order, const UTile *tiles,
                                  uint32_t ntiles, const UClass *classes,
                                  const cfft_launch::dc64 *tw_block, uint32_t *counter,

@@ -162,7 +162,9 @@ hipError_t upload_schedule(DevSchedule &d, const std::vector<UJob> &jobs, const 
       e = hipMemcpy(d.tw_r16, blk.data(), blk.size() * sizeof(dc64), hipMemcpyHostToDevice);
   }
   if (e == hipSuccess) e = upload(&d.classes, classes);
-  if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&d.counter), cfft_ub::kCounterBytes);
+  // the queues' words are zero between launches
+  if (e == hipSuccess)
+    e = upload(&d.counter, std::vector<uint32_t>(cfft_ub::kCounterBytes / sizeof(uint32_t), 0u));
   d.ntiles = (uint32_t)h.tiles.size();
   d.ntiles_r16 = h.ntiles_r16;
   return e;
