@@ -14,14 +14,14 @@
 // Kernel 2: per product and weight k, the inverse program's first pass reads
 // sum_{i+j=k} F[a_i] F[b_j] (i ascending), the last pass untwists, rounds to
 // an integer and accumulates 2^(16 k) D_k into C (owned by one workgroup).
-// Dif16 plans at N = 2048 and 4096 have register-resident forms below (one
-// fused kernel at N = 2048).
+// Dif16 plans at N = 512 ... 4096 have register-resident forms below (one fused
+// kernel up to N = 2048).
 #include <hip/hip_runtime.h>
 
 #include "lds_attr.hpp"
 
 #include "launch.hpp"
-#include "r16_exec.hpp"
+#include "r16s_exec.hpp"
 #include "stockham_exec.hpp"
 
 using namespace cfft_dev;
@@ -40,6 +40,8 @@ __device__ __forceinline__ int64_t limb16(uint64_t v, uint32_t li) {
   return (int64_t)((e >> (16 * li)) & 0xffffu) - 32768;
 }
 
+constexpr double kMagic = 6755399441055744.0;  // 1.5 2^52
+
 // Nearest integer of x (|x| < 2^51) as a two's-complement u64, and the
 // distance |x - that integer|: x + 1.5 2^52 lies in [2^52, 2^53), where the
 // spacing is 1, so the addition rounds x to an integer (half to even) in the
@@ -47,7 +49,6 @@ __device__ __forceinline__ int64_t limb16(uint64_t v, uint32_t li) {
 // integer.  (Differs from round-half-away only at exact half-integers, where
 // the distance is 1/2 and the product's margin reports it.)
 __device__ __forceinline__ uint64_t nearest_u64(double x, double &dist) {
-  constexpr double kMagic = 6755399441055744.0;  // 1.5 2^52
   const double xm = x + kMagic;
   dist = fabs(x - (xm - kMagic));
   return __builtin_bit_cast(uint64_t, xm) - __builtin_bit_cast(uint64_t, kMagic);
@@ -138,143 +139,209 @@ __global__ void __launch_bounds__(512) k_exact_inv(const c64 *__restrict__ F,
   }
 }
 
-// ---- register-resident form for Dif16 plans with n = 1024 (N = 2048) ----
-// One fused kernel, two products per 8-wave workgroup sharing the twiddle
-// block staged in LDS.  Forward: one wave per (product, limb index i)
-// transforms a_i and b_i together (wave-local Dif16 schedule, twiddles
-// shared).  The product's four waves then meet in their exchange buffers,
-// half of the slots at a time, and each lane forms the four weight spectra
-// W_k = sum_{i<=k} F[a_i] F[b_{k-i}] (i ascending) of one point of each
-// product, keeping them (two halves x two products x four weights) in
-// registers until every limb spectrum is read; then it writes them into the
-// exchange buffers, W_k of product pp into wave 4 pp + k's buffer at its
-// point index.  Inverse: wave 4 pp + k transforms W_k back from LDS, rounds,
-// shifts by 16 k and leaves its parts in its buffer; after a barrier the
-// product's first wave sums the four buffers mod 2^64.  No scratch.
+// ---- wave-local form for Dif16 plans with n = 256, 512 and 1024 (N = 512 ... 2048) ----
+// One fused kernel without a scratch: 8-wave workgroups that loop over groups
+// of 2 G products (G = 1, 2, 4 transforms of 1024, 512, 256 points per wave).
+// Wave 4 h + i holds limb i of the G products of half h.  It transforms their
+// a_i and b_i together; the limb spectra meet in the exchange buffers, half of
+// the slots at a time, where each thread forms the four weight spectra
+// W_k = sum_{i<=k} F[a_i] F[b_{k-i}] of two points and keeps them in registers
+// until every limb spectrum is read, then writes W_k into the buffer that held
+// limb k; wave 4 h + k transforms W_k back, rounds, shifts by 16 k and leaves
+// its words in its buffer; all threads add the four words of eight coefficients
+// and store.
+//
+// Tables are staged once per workgroup, words are taken apart with three
+// operations, the integers stay offset by the rounding constant until the four
+// weights are added, and the rounding distance is only formed when the caller
+// asks for the margin.
+//
+// What bounds it: a round (two products of N = 2048, 24 transforms) takes 19.5
+// us, of which LDS traffic is about 9 and VALU issue about 10; the barriers
+// keep the waves in the same phase, so they add up.  Two 4-wave workgroups per
+// CU (twist from global memory) took 81.0 us for 2048 products against 78.4;
+// requesting the next round's words during the inverse or the sums 79-81.
+// Before (us): N = 2048, 2048 products 88 -> 78.4, 64 products 22.1 -> 14.5, one
+// 16.1 -> 13.7 (one workgroup per two products, tables staged by each, generic
+// limbs); on the two-kernel form N = 1024, 4096 products 373 -> 75, one 40 ->
+// 13; N = 512, 8192 products 319 -> 72.
 constexpr uint32_t kXW = 8;
 constexpr uint32_t kXTw = 16 * 64 + 16 * 4;
 constexpr size_t kXLds = (kXTw + kXW * R16<10>::lds_words) * sizeof(c64);
 
+// balanced 16-bit limb li (uniform over the wave) of v: with the lower limbs'
+// carries added (half in every lower limb's place) the field at 16 li is the
+// limb, sign-extended
+struct Limb16 {
+  uint64_t add;
+  uint32_t at;
+  bool high;
+};
+__device__ __forceinline__ Limb16 limb16_of(uint32_t li) {
+  return {0x800080008000ull & (((uint64_t)1 << (16 * li)) - 1), 16 * (li & 1), li >= 2};
+}
+__device__ __forceinline__ int32_t limb16(const Limb16 &f, uint64_t v) {
+  const uint64_t s = v + f.add;
+  return __builtin_amdgcn_sbfe((int32_t)(f.high ? (uint32_t)(s >> 32) : (uint32_t)s), f.at, 16);
+}
+
+template <int LB>
+struct XGeom {
+  static constexpr uint32_t n = 1u << LB, T = n / 16, G = 64 / T;
+  static constexpr uint32_t PW = 2 * G;  // products per workgroup and round
+  static constexpr uint32_t head = kSTw + n;
+  static constexpr size_t lds = (head + kXW * 1024) * sizeof(c64) + kXW * G * sizeof(double);
+  static_assert(lds <= 160 * 1024, "one workgroup per CU");
+};
+
+template <int LB, bool MARGIN>
 __global__ void __launch_bounds__(64 * kXW) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_exact_r16(const uint64_t *__restrict__ A, const uint64_t *__restrict__ B,
-            uint64_t *__restrict__ C, double *margin, uint64_t batch,
-            const c64 *__restrict__ tw_r16, const c64 *__restrict__ twist) {
-  using S = R16<10>;
-  constexpr uint32_t n = S::n;
+k_exact_wave(const uint64_t *__restrict__ A, const uint64_t *__restrict__ B,
+             uint64_t *__restrict__ C, double *margin, uint64_t batch, uint32_t pw,
+             const c64 *__restrict__ tw_blk, const c64 *__restrict__ twist) {
+  using S = R16<LB>;
+  using X = XGeom<LB>;
+  constexpr uint32_t n = X::n, T = X::T, G = X::G;
   extern __shared__ c64 smem[];
-  c64 *ltw = smem;
-  for (uint32_t i = threadIdx.x; i < kXTw; i += blockDim.x) ltw[i] = tw_r16[i];
-  double *s_worst = reinterpret_cast<double *>(smem + kXTw + kXW * S::lds_words);
-  __syncthreads();
+  c64 *ltw = smem, *ltz = smem + kSTw, *xs = smem + X::head;
+  double *s_worst = reinterpret_cast<double *>(xs + kXW * 1024);
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint32_t pp = wave >> 2, li = wave & 3;  // product in the workgroup; limb, then weight
-  const uint64_t p = (uint64_t)blockIdx.x * 2 + pp;
-  const bool active = p < batch;  // every wave reaches the barriers below
-  c64 *x = smem + kXTw + wave * S::lds_words;
-  const uint32_t l = threadIdx.x & 63u;
-  c64 fa[16], fb[16];
-  if (active) {
-    const uint64_t *a = A + p * (2 * n);
-    const uint64_t *b = B + p * (2 * n);
+  const uint32_t li = wave & 3;
+  const uint32_t sub = (threadIdx.x & 63u) / T;
+  const uint32_t pp = (wave >> 2) * G + sub;  // product in the round
+  c64 *x = xs + wave * 1024 + sub * n;
+  auto buffer = [&](uint32_t product, uint32_t limb) {
+    return xs + ((product / G) * 4 + limb) * 1024 + (product % G) * n;
+  };
+  // words of one operand of this lane group's product in the round at g0 (past
+  // the batch in a wave that has a product: the L2-resident twist table's)
+  auto fetch = [&](const uint64_t *src, uint64_t g0, uint64_t *r) {
+    const uint32_t l = launder_u32(threadIdx.x) & (T - 1);
+    const uint64_t p = g0 + pp;
+    const uint64_t *s = p < batch ? src + p * (2ull * n) : reinterpret_cast<const uint64_t *>(twist);
+    s += l;
 #pragma unroll
     for (uint32_t m = 0; m < 16; ++m) {
-      const uint32_t j = l + S::T * m;
-      const c64 z = twist[j];
-      fa[m] = cmul(z, mk((double)(int32_t)limb16(ld_stream(&a[j]), li),
-                         (double)(int32_t)limb16(ld_stream(&a[j + n]), li)));
-      fb[m] = cmul(z, mk((double)(int32_t)limb16(ld_stream(&b[j]), li),
-                         (double)(int32_t)limb16(ld_stream(&b[j + n]), li)));
+      r[2 * m] = ld_stream(&s[T * m]);
+      r[2 * m + 1] = ld_stream(&s[T * m + n]);
     }
-    r16w_transform<true, 2>(fa, fb, x, l, ltw);
-  }
-  const c64 *xs = smem + kXTw;
-  const uint32_t t = threadIdx.x;
-  c64 wq[2][2][4];  // [half][product][weight] at this thread's point of the half
+  };
+  uint64_t g0 = (uint64_t)blockIdx.x * pw;
+  for (uint32_t i = threadIdx.x; i < kSTw; i += 64 * kXW) ltw[i] = tw_blk[r16s_block_index(i)];
+  for (uint32_t i = threadIdx.x; i < n; i += 64 * kXW) ltz[i] = twist[i];
+  __syncthreads();
+  for (; g0 < batch; g0 += (uint64_t)gridDim.x * pw) {
+    const uint32_t l = launder_u32(threadIdx.x) & (T - 1);
+    // a wave without a product skips the work, not the barriers
+    const bool on = (wave >> 2) * G < pw && g0 + (wave >> 2) * G < batch;
+    {
+      c64 fa[16], fb[16];
+      if (on) {
+        uint64_t ra[32], rb[32];
+        fetch(A, g0, ra);
+        fetch(B, g0, rb);
+        sched_fence();
+        const Limb16 f = limb16_of(li);
 #pragma unroll
-  for (uint32_t h = 0; h < 2; ++h) {
-    wave_lds_fence();
-    if (active) {
+        for (uint32_t m = 0; m < 16; ++m) {
+          const c64 z = ltz[l + T * m];
+          fa[m] = cmul(z, mk((double)limb16(f, ra[2 * m]), (double)limb16(f, ra[2 * m + 1])));
+          fb[m] = cmul(z, mk((double)limb16(f, rb[2 * m]), (double)limb16(f, rb[2 * m + 1])));
+        }
+        r16s_transform<LB, true, 2>(fa, fb, x, l, ltw);
+      }
+      const uint32_t t = launder_u32(threadIdx.x);
+      c64 wq[2][2][4];  // [half][e][weight] at this thread's points of the half
 #pragma unroll
-      for (uint32_t s = 0; s < 8; ++s) {
-        x[s * 64 + l] = fa[8 * h + s];
-        x[512 + s * 64 + l] = fb[8 * h + s];
+      for (uint32_t h = 0; h < 2; ++h) {
+        wave_lds_fence();
+        if (on) {
+#pragma unroll
+          for (uint32_t s = 0; s < 8; ++s) {
+            x[s * T + l] = fa[8 * h + s];
+            x[n / 2 + s * T + l] = fb[8 * h + s];
+          }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t e = 0; e < 2; ++e) {
+          const uint32_t at = t + 512 * e, q2 = at / (n / 2), pt = at % (n / 2);
+          c64 wa[4], wb[4];
+#pragma unroll
+          for (uint32_t i = 0; i < 4; ++i) {
+            const c64 *y = buffer(q2, i) + pt;
+            wa[i] = y[0];
+            wb[i] = y[n / 2];
+          }
+#pragma unroll
+          for (uint32_t k = 0; k < 4; ++k) {
+            c64 d = cmul(wa[0], wb[k]);
+#pragma unroll
+            for (uint32_t i = 1; i <= k; ++i) {
+              d.re = __fma_rn(wa[i].re, wb[k - i].re, __fma_rn(-wa[i].im, wb[k - i].im, d.re));
+              d.im = __fma_rn(wa[i].re, wb[k - i].im, __fma_rn(wa[i].im, wb[k - i].re, d.im));
+            }
+            wq[h][e][k] = d;
+          }
+        }
+        __syncthreads();  // every limb spectrum of the half read
+      }
+#pragma unroll
+      for (uint32_t h = 0; h < 2; ++h)
+#pragma unroll
+        for (uint32_t e = 0; e < 2; ++e) {
+          const uint32_t at = t + 512 * e, q2 = at / (n / 2), pt = at % (n / 2);
+          const uint32_t q = (pt & (T - 1)) + T * S::end_m(8 * h + pt / T);
+#pragma unroll
+          for (uint32_t k = 0; k < 4; ++k) buffer(q2, k)[q] = wq[h][e][k];
+        }
+    }
+    __syncthreads();
+    // inverse of W_k, k = li: 2^(16 k) D_k, rounded and still offset
+    if (on) {
+      c64 v[16];
+#pragma unroll
+      for (uint32_t m = 0; m < 16; ++m) v[m] = x[l + T * m];
+      r16s_transform<LB, false, 1>(v, v, x, l, ltw);
+      uint64_t *xb = reinterpret_cast<uint64_t *>(x);
+      double worst = 0.0;
+#pragma unroll
+      for (uint32_t s = 0; s < 16; ++s) {
+        const c64 tz = ltz[l + T * S::end_m(s)];
+        const c64 r = cmul(mk(tz.re * (1.0 / n), (-tz.im) * (1.0 / n)), v[s]);
+        const double x0 = r.re + kMagic, x1 = r.im + kMagic;
+        if constexpr (MARGIN)
+          worst = fmax(worst, fmax(fabs(r.re - (x0 - kMagic)), fabs(r.im - (x1 - kMagic))));
+        xb[2 * s * T + l] = __builtin_bit_cast(uint64_t, x0) << (16 * li);
+        xb[(2 * s + 1) * T + l] = __builtin_bit_cast(uint64_t, x1) << (16 * li);
+        if ((s & 3) == 3) sched_fence();
+      }
+      if constexpr (MARGIN) {
+        for (uint32_t off = 1; off < T; off <<= 1)
+          worst = fmax(worst, __shfl_xor(worst, (int)off));
+        if (l == 0) s_worst[pp * 4 + li] = worst;
       }
     }
     __syncthreads();
+    constexpr uint64_t kOffset = __builtin_bit_cast(uint64_t, kMagic);
+    constexpr uint64_t kOffsets =
+        kOffset + (kOffset << 16) + (kOffset << 32) + (kOffset << 48);
+    const uint32_t t = launder_u32(threadIdx.x);
 #pragma unroll
-    for (uint32_t q2 = 0; q2 < 2; ++q2) {
-      c64 wa[4], wb[4];
+    for (uint32_t e = 0; e < 8; ++e) {
+      const uint32_t at = t + 512 * e, q2 = at / (2 * n), r = at % (2 * n);
+      const uint32_t q = r / T, j = (r & (T - 1)) + T * S::end_m(q >> 1) + (q & 1 ? n : 0);
+      uint64_t sum = 0 - kOffsets;
 #pragma unroll
-      for (uint32_t i = 0; i < 4; ++i) {
-        wa[i] = xs[(4 * q2 + i) * S::lds_words + t];
-        wb[i] = xs[(4 * q2 + i) * S::lds_words + 512 + t];
-      }
-#pragma unroll
-      for (uint32_t k = 0; k < 4; ++k) {
-        c64 d = cmul(wa[0], wb[k]);
-#pragma unroll
-        for (uint32_t i = 1; i <= k; ++i) d = cadd(d, cmul(wa[i], wb[k - i]));
-        wq[h][q2][k] = d;
-      }
+      for (uint32_t k = 0; k < 4; ++k) sum += reinterpret_cast<const uint64_t *>(buffer(q2, k))[r];
+      if (q2 < pw && g0 + q2 < batch) st_stream(sum, &C[(g0 + q2) * (2ull * n) + j]);
     }
-    __syncthreads();  // every limb spectrum of the half read
-  }
-  // W_k of product q2, point q, to wave 4 q2 + k's buffer at q
-#pragma unroll
-  for (uint32_t h = 0; h < 2; ++h) {
-    const uint32_t q = (t & 63) + S::T * S::end_m(8 * h + (t >> 6));
-#pragma unroll
-    for (uint32_t q2 = 0; q2 < 2; ++q2)
-#pragma unroll
-      for (uint32_t k = 0; k < 4; ++k) smem[kXTw + (4 * q2 + k) * S::lds_words + q] = wq[h][q2][k];
-  }
-  __syncthreads();
-  // inverse of W_k, k = li: 2^(16 k) D_k, rounded
-  const uint32_t k = li;
-  const double inv_n = 1.0 / (double)n;
-  double worst = 0.0;
-  uint64_t part[32];
-  {
-    c64 v[16];
-#pragma unroll
-    for (uint32_t m = 0; m < 16; ++m) v[m] = x[l + S::T * m];
-    r16w_transform<false, 1>(v, v, x, l, ltw);
-    const c64 *tws = launder(twist);
-#pragma unroll
-    for (uint32_t s = 0; s < 16; ++s) {
-      const uint32_t j = l + S::T * S::end_m(s);
-      const c64 tz = tws[j];
-      const c64 r = cmul(mk(tz.re * inv_n, (-tz.im) * inv_n), v[s]);
-      double d0, d1;
-      const uint64_t x0 = nearest_u64(r.re, d0), x1 = nearest_u64(r.im, d1);
-      worst = fmax(worst, fmax(d0, d1));
-      part[2 * s] = x0 << (16 * k);
-      part[2 * s + 1] = x1 << (16 * k);
+    if constexpr (MARGIN) {
+      if (t < pw && g0 + t < batch)
+        margin[g0 + t] = fmax(fmax(s_worst[4 * t], s_worst[4 * t + 1]),
+                              fmax(s_worst[4 * t + 2], s_worst[4 * t + 3]));
     }
-  }
-  // the transform's last LDS reads are behind its final wave fence; reuse the
-  // buffer for this wave's 32 words per lane
-  uint64_t *xb = reinterpret_cast<uint64_t *>(x);
-#pragma unroll
-  for (uint32_t q = 0; q < 32; ++q) xb[q * 64 + l] = part[q];
-  for (uint32_t off = 1; off < 64; off <<= 1) worst = fmax(worst, __shfl_xor(worst, (int)off));
-  if (l == 0) s_worst[wave] = worst;
-  __syncthreads();
-  if (active && k == 0) {
-    const uint64_t *b1 = reinterpret_cast<const uint64_t *>(x + 1 * S::lds_words);
-    const uint64_t *b2 = reinterpret_cast<const uint64_t *>(x + 2 * S::lds_words);
-    const uint64_t *b3 = reinterpret_cast<const uint64_t *>(x + 3 * S::lds_words);
-    uint64_t *c = C + p * (2 * n);
-#pragma unroll
-    for (uint32_t s = 0; s < 16; ++s) {
-      const uint32_t j = l + S::T * S::end_m(s);
-      const uint32_t q0 = (2 * s) * 64 + l, q1 = (2 * s + 1) * 64 + l;
-      st_stream(part[2 * s] + b1[q0] + b2[q0] + b3[q0], &c[j]);
-      st_stream(part[2 * s + 1] + b1[q1] + b2[q1] + b3[q1], &c[j + n]);
-    }
-    if (margin && l == 0)
-      margin[p] = fmax(fmax(s_worst[wave], s_worst[wave + 1]),
-                       fmax(s_worst[wave + 2], s_worst[wave + 3]));
+    __syncthreads();  // the buffers are read
   }
 }
 
@@ -496,6 +563,32 @@ hipError_t launch_e(const Program &fwd, const Program &inv, const uint64_t *a, c
   return hipGetLastError();
 }
 
+template <int LB, bool MARGIN>
+hipError_t launch_wave_m(const uint64_t *a, const uint64_t *b, uint64_t *c, double *margin,
+                         uint64_t batch, const c64 *tw_blk, const c64 *twist, hipStream_t s) {
+  using X = XGeom<LB>;
+  int cus = 0;
+  hipError_t e = cfft_launch::cu_count(&cus);
+  if (e == hipSuccess)
+    e = cfft_launch::ensure_lds(reinterpret_cast<const void *>(k_exact_wave<LB, MARGIN>), X::lds);
+  if (e != hipSuccess) return e;
+  // half of the waves' places while that gives every group of G products a CU
+  // of its own (N = 2048, 64 products: 20.4 -> 14.5 us)
+  const uint32_t pw = batch <= (uint64_t)cus * X::G ? X::G : X::PW;
+  const uint64_t groups = (batch + pw - 1) / pw;
+  const uint32_t grid = (uint32_t)(groups < (uint64_t)cus ? groups : (uint64_t)cus);
+  hipLaunchKernelGGL((k_exact_wave<LB, MARGIN>), dim3(grid), dim3(64 * kXW), X::lds, s, a, b, c,
+                     margin, batch, pw, tw_blk, twist);
+  return hipGetLastError();
+}
+
+template <int LB>
+hipError_t launch_wave(const uint64_t *a, const uint64_t *b, uint64_t *c, double *margin,
+                       uint64_t batch, const c64 *tw_blk, const c64 *twist, hipStream_t s) {
+  return margin ? launch_wave_m<LB, true>(a, b, c, margin, batch, tw_blk, twist, s)
+                : launch_wave_m<LB, false>(a, b, c, margin, batch, tw_blk, twist, s);
+}
+
 }  // namespace
 
 namespace cfft_launch {
@@ -518,22 +611,20 @@ hipError_t exact_polymul(const Program &fwd, const Program &inv, const uint64_t 
   }
 }
 
-// Register-resident form: Dif16 plan with n = 1024; tw_r16 is the plan's
-// lane-major twiddle block.  One fused kernel, two products per workgroup,
-// no scratch.
-hipError_t exact_polymul_r16(const uint64_t *a, const uint64_t *b, uint64_t *c, double *margin,
-                             uint64_t batch, const dc64 *tw_r16, const dc64 *twist,
-                             hipStream_t s) {
+// Wave-local form: Dif16 plans with n = base_n = 256, 512 and 1024 (log2n 8, 9,
+// 10); tw_blk is the 1024-point r16 block.  One persistent launch, no scratch.
+hipError_t exact_polymul_wave(uint32_t log2n, const uint64_t *a, const uint64_t *b, uint64_t *c,
+                              double *margin, uint64_t batch, const dc64 *tw_blk,
+                              const dc64 *twist, hipStream_t s) {
   if (batch == 0) return hipSuccess;
-  constexpr size_t lds = kXLds + kXW * sizeof(double);  // + each wave's margin
-  hipError_t e = cfft_launch::ensure_lds(reinterpret_cast<const void *>(k_exact_r16), lds);
-  if (e != hipSuccess) return e;
-  const c64 *t = reinterpret_cast<const c64 *>(tw_r16);
+  const c64 *t = reinterpret_cast<const c64 *>(tw_blk);
   const c64 *z = reinterpret_cast<const c64 *>(twist);
-  const uint64_t per_wg = kXW / 4;  // products per workgroup (4 waves each)
-  hipLaunchKernelGGL(k_exact_r16, dim3((uint32_t)((batch + per_wg - 1) / per_wg)), dim3(64 * kXW),
-                     lds, s, a, b, c, margin, batch, t, z);
-  return hipGetLastError();
+  switch (log2n) {
+    case 8: return launch_wave<8>(a, b, c, margin, batch, t, z, s);
+    case 9: return launch_wave<9>(a, b, c, margin, batch, t, z, s);
+    case 10: return launch_wave<10>(a, b, c, margin, batch, t, z, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 // Wave-local form: Dif16 plan with n = 2048 and base_n = 1024; tw is the

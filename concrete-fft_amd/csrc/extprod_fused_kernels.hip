@@ -33,7 +33,7 @@
 #include "gadget.hpp"
 #include "launch.hpp"
 #include "lds_attr.hpp"
-#include "r16_exec.hpp"
+#include "r16s_exec.hpp"
 
 using namespace cfft_dev;
 using cfft_launch::dc64;
@@ -41,8 +41,6 @@ using cfft_launch::dc64;
 namespace {
 
 constexpr uint32_t kFWaves = 8;
-// the 1024-point r16 twiddle block's rows k = 1 ... 15 (T[k l], then T[16 k p])
-constexpr uint32_t kFTw1 = 15 * 64, kFTw = kFTw1 + 15 * 4;
 
 template <int LOG2N>
 struct FGeom {
@@ -55,38 +53,10 @@ struct FGeom {
   static constexpr uint32_t PB = nb / (64 * kFWaves);  // points per thread and chunk
   // the twist table, or at n = 2048 its entries 0 ... 1024 (twist_point)
   static constexpr uint32_t zw = n <= 1024 ? n : 1025;
-  static constexpr uint32_t head = kFTw + zw;
+  static constexpr uint32_t head = kSTw + zw;
   static constexpr size_t lds = (size_t)(head + U * nb) * sizeof(c64);
   static_assert(lds <= 160 * 1024, "one workgroup per CU");
 };
-
-// One base transform of 2^LB points (LB = 9, 10) on T = 2^LB / 16 lanes:
-// r16l_transform with the twiddle rows k >= 1 only (`tw`, kFTw entries) and an
-// exchange buffer of exactly 2^LB points, point i at i ^ ((i >> 4) & 15), as
-// in r16x_transform.
-template <int LB, bool FWD>
-__device__ __forceinline__ void base_transform(c64 *v, c64 *x, uint32_t l, const c64 *tw) {
-  using S = R16<LB>;
-  constexpr uint32_t cs = 1u << (10 - LB);  // column stride in the 1024-point block
-  const uint32_t p = l >> 4, q = l & 15;
-  butterfly<16, FWD>(v);
-  sched_fence();
-  twiddle_rows_x2<FWD>(v, v, 1, tw, 64, l * cs);
-  wave_lds_fence();
-#pragma unroll
-  for (int k = 0; k < 16; ++k) x[16 * l + ((uint32_t)k ^ q)] = v[k];
-  wave_lds_fence();
-#pragma unroll
-  for (int k = 0; k < 16; ++k)
-    v[k] = x[S::T * (uint32_t)k + 16 * p + (q ^ ((p + S::T / 16 * (uint32_t)k) & 15))];
-  wave_lds_fence();  // last use of x
-  butterfly<16, FWD>(v);
-  sched_fence();
-  twiddle_rows_x2<FWD>(v, v, 1, tw + kFTw1, 4, p * cs);
-  r16_exchange2_rows<LB>(v);
-#pragma unroll
-  for (uint32_t i = 0; i < S::NB; ++i) butterfly<S::REND, FWD>(v + i * S::REND);
-}
 
 // Twist factor of point i of chunk ch.  zeta_j = exp(i pi j / 2n), so that at
 // n = 2048 the second chunk's factors are the first one's mirrored at j =
@@ -134,7 +104,7 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
   constexpr uint32_t RG = F::U / CH / P;  // rows of one GLWE in a round
   static_assert(RG >= 1 && P * K1 * CH <= F::U, "the columns must fit the units");
   extern __shared__ c64 smem[];
-  c64 *ltw = smem, *ltz = smem + kFTw, *xs = smem + F::head;
+  c64 *ltw = smem, *ltz = smem + kSTw, *xs = smem + F::head;
   const uint32_t rows = K1 * levels;
   const uint32_t tid = threadIdx.x;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -171,11 +141,9 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
   {
     // the twiddle block's loads, then the first coefficients', in flight together
     // (rows k = 1 ... 15 start at 64 and at 1024 + 4 in the plan's block)
-    static_assert(kFTw > 512 && kFTw <= 1024, "two entries per thread");
+    static_assert(kSTw > 512 && kSTw <= 1024, "two entries per thread");
     const auto blk = point_buffer(tw_blk, 16 * 64 + 16 * 4), zt = point_buffer(twist, n);
-    auto entry = [&](uint32_t i) {
-      return load_point(blk, i < kFTw1 ? 64 + i : 1024 + 4 + (i - kFTw1));
-    };
+    auto entry = [&](uint32_t i) { return load_point(blk, r16s_block_index(i)); };
     const c64 t0 = entry(tid), t1 = entry(tid + 512);
     // (n = 512: one twist entry per thread; n = 2048: entry 1024 as well)
     const c64 z0 = load_point(zt, tid), z1 = load_point(zt, F::zw > 512 ? tid + 512 : n);
@@ -183,7 +151,7 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
     fetch(g0, 0);
     sched_fence();
     ltw[tid] = t0;
-    if (tid + 512 < kFTw) ltw[tid + 512] = t1;
+    if (tid + 512 < kSTw) ltw[tid + 512] = t1;
     ltz[tid] = z0;
     if constexpr (F::zw > 512) ltz[tid + 512] = z1;
     if (F::zw > 1024 && tid == 0) ltz[1024] = z2;
@@ -288,7 +256,7 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
         sched_fence();
       }
       if (on) {
-        base_transform<F::LB, true>(v, x, l, ltw);
+        r16s_transform<F::LB, true, 1>(v, v, x, l, ltw);
         wave_lds_fence();
 #pragma unroll
         for (uint32_t s = 0; s < 16; ++s) x[s * T + l] = v[s];
@@ -350,7 +318,7 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
     if (busy) {
 #pragma unroll
       for (uint32_t m = 0; m < 16; ++m) v[m] = x[l + T * m];
-      base_transform<F::LB, false>(v, x, l, ltw);
+      r16s_transform<F::LB, false, 1>(v, v, x, l, ltw);
     }
     // untwist = conj(twist) / n (an exact scaling: the plan's untwist table)
     auto put = [&](uint64_t *o, uint32_t c2, uint32_t i, c64 y) {

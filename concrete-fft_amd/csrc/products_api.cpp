@@ -21,9 +21,9 @@ hipError_t exact_polymul(const cfft_prog::Program &fwd, const cfft_prog::Program
 hipError_t exact_polymul_w2(const uint64_t *a, const uint64_t *b, uint64_t *c, double *margin,
                             uint64_t batch, const dc64 *tw, const dc64 *tw_blk,
                             const dc64 *twist, const dc64 *untwist, dc64 *F, hipStream_t s);
-hipError_t exact_polymul_r16(const uint64_t *a, const uint64_t *b, uint64_t *c, double *margin,
-                             uint64_t batch, const dc64 *tw_r16, const dc64 *twist,
-                             hipStream_t s);
+hipError_t exact_polymul_wave(uint32_t log2n, const uint64_t *a, const uint64_t *b, uint64_t *c,
+                              double *margin, uint64_t batch, const dc64 *tw_blk,
+                              const dc64 *twist, hipStream_t s);
 hipError_t torus_to_fourier(const cfft_prog::Program &fwd, const uint64_t *key, dc64 *out,
                             uint64_t npolys, const dc64 *tw, const dc64 *twist, hipStream_t s);
 hipError_t external_product_split(const cfft_prog::Program &fwd, const cfft_prog::Program &inv,
@@ -197,10 +197,13 @@ int cfft_exact_polymul_u64(cfft_plan plan, const uint64_t *a, const uint64_t *b,
   if (plan->n < 2 || plan->n > 2048 || plan->fwd_full.npass == 0)
     return set_error(CFFT_ERROR_SIZE, "exact product supports 4 <= N <= 4096 (fft_size <= 2048)");
   hipStream_t s = (hipStream_t)stream;
-  // Dif16 with base_n == n == 1024: one fused kernel, no scratch
-  if (plan->n == 1024 && plan->d_tw_r16)
-    return hip_error(cfft_launch::exact_polymul_r16(a, b, c, margin, batch, plan->d_tw_r16,
-                                                    plan->d_twist, s),
+  // Dif16 with base_n == n = 256, 512, 1024: one fused kernel, no scratch
+  const cfft_launch::dc64 *blk = plan->n == 1024 ? plan->d_tw_r16
+                                 : plan->n < 1024 && plan->base_n == plan->n ? plan->d_tw_base1024
+                                                                             : nullptr;
+  if (blk)
+    return hip_error(cfft_launch::exact_polymul_wave(ilog2(plan->n), a, b, c, margin, batch, blk,
+                                                     plan->d_twist, s),
                      "exact product");
   // the wave-local form keeps the 4 weight spectra of a product, the generic
   // form its 8 limb spectra

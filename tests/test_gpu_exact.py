@@ -153,3 +153,33 @@ def test_exact_worst_case_limbs(cfft, oracle, N, base_n):
     assert np.array_equal(c, oracle.schoolbook_u64(a, b))
     # exact while < 1/2; measured 0.0098 at N = 4096, so wide headroom remains
     assert 0.0 <= margin.max() < 2.0 ** -5, margin
+
+
+@pytest.mark.parametrize("N", [512, 1024, 2048])
+@pytest.mark.parametrize("batch", [1, 2, 7, 8, 9, 2065])
+def test_exact_wave_groups(cfft, oracle, N, batch):
+    """The fused kernel of Dif16 plans (8, 4 or 2 products per workgroup and
+    round at N = 512, 1024, 2048; at most one workgroup per CU): groups partly
+    filled, a second and later round, with and without the margin."""
+    from cfft_amd import products
+    from cfft_amd.unordered import FftAlgo, Method, Plan
+    print("exact wave: N=%d batch=%d" % (N, batch), flush=True)
+    rng = np.random.default_rng(N + batch)
+    a = rng.integers(0, M, (batch, N), dtype=np.uint64)
+    b = rng.integers(0, M, (batch, N), dtype=np.uint64)
+    a[0, :4] = [0, M - 1, 1 << 63, 0x7fff7fff7fff7fff]
+    a[batch - 1] = 0x8000800080008000  # every limb -2^15
+    b[batch - 1] = 0x8000800080008000
+    plan = Plan(N // 2, Method.UserProvided(FftAlgo.Dif16, N // 2))
+    c = products.exact_polymul_u64_host(plan, a, b)
+    cm, margin = products.exact_polymul_u64_host(plan, a, b, with_margin=True)
+    assert np.array_equal(c, cm) and margin.shape == (batch,)
+    # |D_3| <= 4 N 2^30 = 2^43 at N = 2048: a relative error of 2^-52 log2(N)
+    # leaves the rounded sums within 11 * 2^-9 of an integer
+    assert 0 < margin.max() < 11 * 2.0**-9
+    for i in sorted({0, batch // 2, batch - 1}):
+        want = oracle.schoolbook_u64(a[i:i + 1], b[i:i + 1])[0]
+        assert np.array_equal(c[i], want), (i, int(np.sum(c[i] != want)))
+    for i in range(0, batch, 500):
+        part = products.exact_polymul_u64_host(plan, a[i:i + 1], b[i:i + 1])
+        assert np.array_equal(part[0], c[i]), i
