@@ -126,60 +126,54 @@ __device__ __forceinline__ uint32_t group_pos(uint32_t g, uint32_t ptop, uint32_
   return base + off;
 }
 
-// One round of R stages on NG = 8 / R-point groups per thread.
-// FWD: stages st0, st0+1, .. (bit ptop = Lg-1-st0 downwards), CT butterflies.
-// INV: stages processed from the low bit up, GS butterflies.
+// The 2^R - 1 twiddles of a group's round: stage b of the round (pair bit
+// p = ptop - b, twiddle index 2^(Lg-1-p) + (position >> (p + 1))) has one for
+// each value c of the round's bits above p, at w[2^b - 1 + c].
+template <int R>
+__device__ __forceinline__ void round_twiddles(cdd *w, uint32_t g, uint32_t ptop, uint32_t Lg,
+                                               uint32_t jhi, const Tw &tw) {
+  const uint32_t base = jhi | group_pos<R>(g, ptop, 0);
+#pragma unroll
+  for (int b = 0; b < R; ++b) {
+    const uint32_t p = ptop - (uint32_t)b;
+#pragma unroll
+    for (int c = 0; c < (1 << b); ++c)
+      w[(1 << b) - 1 + c] =
+          load_tw(tw, (1u << (Lg - 1 - p)) + ((base | ((uint32_t)c << (p + 1))) >> (p + 1)));
+  }
+}
+
+// One round of R stages on a group of 2^R points (its twiddles in w).
+// FWD: from the top pair bit down, CT butterflies.
+// INV: from the low bit up, GS butterflies.
 // Positions are local to a block of 2^L points that starts at point jhi of a
 // transform of 2^Lg points (jhi = 0, Lg = L for a whole transform); stage
 // indices and twiddles are those of the whole transform.
 template <int R, bool FWD, int MULV>
-__device__ __forceinline__ void round_regs(cdd *z, uint32_t g, uint32_t ptop, uint32_t Lg,
-                                           uint32_t jhi, const Tw &tw) {
+__device__ __forceinline__ void round_regs(cdd *z, const cdd *w) {
   // z[u], u < 2^R, indexed with the bit for position ptop-b at bit (R-1-b)
-  const uint32_t base = group_pos<R>(g, ptop, 0);
-  if (FWD) {
 #pragma unroll
-    for (int b = 0; b < R; ++b) {
-      const uint32_t p = ptop - (uint32_t)b;       // pair bit
-      const uint32_t st = Lg - 1 - p;              // stage index, m = 2^st
+  for (int s = 0; s < R; ++s) {
+    const int b = FWD ? s : R - 1 - s;
 #pragma unroll
-      for (int u = 0; u < (1 << R); ++u) {
-        if ((u >> (R - 1 - b)) & 1) continue;
-        const int v = u | (1 << (R - 1 - b));
-        uint32_t j = base;
-#pragma unroll
-        for (int c = 0; c < R; ++c) j |= ((uint32_t)(u >> (R - 1 - c)) & 1u) << (ptop - c);
-        const uint32_t i = (jhi | j) >> (p + 1);
-        const cdd w = load_tw(tw, (1u << st) + i);
-        const cdd z1w = cmul<MULV>(z[v], w);
-        const cdd z0 = z[u];
+    for (int u = 0; u < (1 << R); ++u) {
+      if ((u >> (R - 1 - b)) & 1) continue;
+      const int v = u | (1 << (R - 1 - b));
+      const cdd wu = w[(1 << b) - 1 + (u >> (R - b))];
+      const cdd z0 = z[u], z1 = z[v];
+      if (FWD) {
+        const cdd z1w = cmul<MULV>(z1, wu);
         z[u].re = add_est(z0.re, z1w.re);
         z[u].im = add_est(z0.im, z1w.im);
         z[v].re = sub_est(z0.re, z1w.re);
         z[v].im = sub_est(z0.im, z1w.im);
-      }
-    }
-  } else {
-#pragma unroll
-    for (int b = R - 1; b >= 0; --b) {
-      const uint32_t p = ptop - (uint32_t)b;
-      const uint32_t st = Lg - 1 - p;
-#pragma unroll
-      for (int u = 0; u < (1 << R); ++u) {
-        if ((u >> (R - 1 - b)) & 1) continue;
-        const int v = u | (1 << (R - 1 - b));
-        uint32_t j = base;
-#pragma unroll
-        for (int c = 0; c < R; ++c) j |= ((uint32_t)(u >> (R - 1 - c)) & 1u) << (ptop - c);
-        const uint32_t i = (jhi | j) >> (p + 1);
-        const cdd w = load_tw(tw, (1u << st) + i);
-        const cdd z0 = z[u], z1 = z[v];
+      } else {
         cdd d;
         d.re = sub_est(z0.re, z1.re);
         d.im = sub_est(z0.im, z1.im);
         z[u].re = add_est(z0.re, z1.re);
         z[u].im = add_est(z0.im, z1.im);
-        z[v] = cmul_conj<MULV>(d, w);
+        z[v] = cmul_conj<MULV>(d, wu);
       }
     }
   }
@@ -193,7 +187,11 @@ __device__ __forceinline__ void run_round(double *lds, const Bufs &gbuf, bool fi
   constexpr int NG = 8 / P;
   const uint32_t n = 1u << L;
   const uint32_t pn = pad128(n);
-  cdd z[NG][P];
+  cdd z[NG][P], w[NG][P - 1];
+  // requested before the points: they arrive while those are exchanged
+#pragma unroll
+  for (int q = 0; q < NG; ++q)
+    round_twiddles<R>(w[q], lt + T * (uint32_t)q, ptop, Lg, jhi, tw);
 #pragma unroll
   for (int q = 0; q < NG; ++q) {
     const uint32_t g = lt + T * (uint32_t)q;
@@ -222,7 +220,7 @@ __device__ __forceinline__ void run_round(double *lds, const Bufs &gbuf, bool fi
 #pragma unroll
   for (int q = 0; q < NG; ++q) {
     const uint32_t g = lt + T * (uint32_t)q;
-    round_regs<R, FWD, MULV>(z[q], g, ptop, Lg, jhi, tw);
+    round_regs<R, FWD, MULV>(z[q], w[q]);
 #pragma unroll
     for (int u = 0; u < P; ++u) {
       const uint32_t j = group_pos<R>(g, ptop, (uint32_t)u);
@@ -252,7 +250,7 @@ __device__ __forceinline__ void run_round(double *lds, const Bufs &gbuf, bool fi
 // wave), each with its own LDS slice; a block past the last is idle but
 // takes part in every barrier.
 template <bool FWD, int MULV>
-__global__ void __launch_bounds__(512) k_fft128(double *re0, double *re1, double *im0,
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) k_fft128(double *re0, double *re1, double *im0,
                                                 double *im1, const double *__restrict__ t_re0,
                                                 const double *__restrict__ t_re1,
                                                 const double *__restrict__ t_im0,
@@ -311,7 +309,8 @@ __global__ void __launch_bounds__(256) k_fft128_global(double *re0, double *re1,
   const uint32_t g = (uint32_t)(gid & ((1ull << (Lg - R)) - 1));
   const uint64_t off = tr << Lg;
   Tw tw{t_re0, t_re1, t_im0, t_im1};
-  cdd z[P];
+  cdd z[P], w[P - 1];
+  round_twiddles<R>(w, g, ptop, Lg, 0u, tw);
 #pragma unroll
   for (int u = 0; u < P; ++u) {
     const uint64_t j = off + group_pos<R>(g, ptop, (uint32_t)u);
@@ -320,7 +319,7 @@ __global__ void __launch_bounds__(256) k_fft128_global(double *re0, double *re1,
     z[u].im.hi = im0[j];
     z[u].im.lo = im1[j];
   }
-  round_regs<R, FWD, MULV>(z, g, ptop, Lg, 0u, tw);
+  round_regs<R, FWD, MULV>(z, w);
 #pragma unroll
   for (int u = 0; u < P; ++u) {
     const uint64_t j = off + group_pos<R>(g, ptop, (uint32_t)u);
