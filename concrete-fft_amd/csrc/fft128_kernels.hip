@@ -10,8 +10,8 @@
 //
 // Schedule: one workgroup per transform of n points (4 SoA arrays in LDS,
 // 32 B per point).  The log2(n) radix-2 stages (CT forward
-// src/fft128/mod.rs:351-402, GS inverse :1104-1155) are taken three at a
-// time: each thread owns 8 points that form closed radix-2 networks over those
+// src/fft128/mod.rs:351-402, GS inverse :1104-1155) are taken two at a
+// time: each thread owns 4 points that form closed radix-2 networks over those
 // stages, applies them in registers, and exchanges through LDS between
 // rounds.  The first round reads global memory and the last writes it.
 #include <hip/hip_runtime.h>
@@ -108,9 +108,15 @@ struct Bufs {
 };
 
 __host__ __device__ __forceinline__ uint32_t pad128(uint32_t i) { return i + (i >> 5); }
-// blocks of 2^L points per k_fft128 workgroup: enough to fill one wave
+// Points per k_fft128 thread (2^kRB) and blocks of 2^L points per workgroup:
+// enough to fill one wave.  Double-double sums are serial chains, and a CU's LDS
+// holds 4096 points: four points per thread put 16 waves on it (under 128
+// registers each) where eight put 8, which hides more than the extra exchange
+// costs (us: n = 1024 x 1000 inverse 45.2 -> 37.8, n = 512 x 4096 forward 89.5 ->
+// 65.6, n = 64 x 32768 forward 80.4 -> 56.7).
+constexpr uint32_t kRB = 2;
 __host__ __device__ __forceinline__ uint32_t fft128_blocks_per_wg(uint32_t L) {
-  return L >= 9 ? 1u : 1u << (9 - L);
+  return L >= 6 + kRB ? 1u : 1u << (6 + kRB - L);
 }
 
 // Position of point `u` (3-bit combination, most significant = first stage
@@ -184,7 +190,7 @@ __device__ __forceinline__ void run_round(double *lds, const Bufs &gbuf, bool fi
                                           uint32_t ptop, uint32_t L, uint32_t Lg, uint32_t jhi,
                                           uint32_t lt, uint32_t T, const Tw &tw, bool active) {
   constexpr int P = 1 << R;
-  constexpr int NG = 8 / P;
+  constexpr int NG = (1 << kRB) / P;
   const uint32_t n = 1u << L;
   const uint32_t pn = pad128(n);
   cdd z[NG][P], w[NG][P - 1];
@@ -243,14 +249,14 @@ __device__ __forceinline__ void run_round(double *lds, const Bufs &gbuf, bool fi
   __syncthreads();
 }
 
-// Blocks of n = 2^L points (L >= 3), T = n / 8 threads each: the rounds over
+// Blocks of n = 2^L points (L >= 3), T = n / 4 threads each: the rounds over
 // bits 0 .. L-1 of a transform of 2^Lg points (Lg >= L) whose blocks are
 // contiguous; block b is block b % 2^(Lg-L) of transform b / 2^(Lg-L), at
 // b * n.  A workgroup holds G = max(1, 64 / T) blocks (at least one full
 // wave), each with its own LDS slice; a block past the last is idle but
 // takes part in every barrier.
 template <bool FWD, int MULV>
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) k_fft128(double *re0, double *re1, double *im0,
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) k_fft128(double *re0, double *re1, double *im0,
                                                 double *im1, const double *__restrict__ t_re0,
                                                 const double *__restrict__ t_re1,
                                                 const double *__restrict__ t_im0,
@@ -258,35 +264,36 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))
                                                 uint32_t Lg, uint64_t blocks) {
   extern __shared__ double smem[];
   const uint32_t n = 1u << L;
-  const uint32_t T = n / 8;
+  const uint32_t T = n >> kRB;
   const uint32_t G = fft128_blocks_per_wg(L);
-  const uint32_t sub = threadIdx.x >> (L - 3), lt = threadIdx.x & (T - 1);
+  const uint32_t sub = threadIdx.x >> (L - kRB), lt = threadIdx.x & (T - 1);
   const uint64_t tr = (uint64_t)blockIdx.x * G + sub;
   const bool active = tr < blocks;
   double *lds = smem + (size_t)sub * 4 * pad128(n);
   const uint32_t jhi = (uint32_t)(tr & ((1ull << (Lg - L)) - 1)) << L;
   Bufs g{re0 + tr * n, re1 + tr * n, im0 + tr * n, im1 + tr * n};
   Tw tw{t_re0, t_re1, t_im0, t_im1};
-  const uint32_t rounds = (L + 2) / 3;
+  const uint32_t rounds = (L + kRB - 1) / kRB;
   for (uint32_t r = 0; r < rounds; ++r) {
     const bool first = r == 0, last = r + 1 == rounds;
-    // forward: bits L-1 down to 0 in chunks of 3 from the top;
-    // inverse: bits 0 up to L-1 in chunks of 3 from the bottom
+    // forward: bits L-1 down to 0 in chunks of kRB from the top;
+    // inverse: bits 0 up to L-1 in chunks of kRB from the bottom
     uint32_t lo_bit, nb;
     if (FWD) {
-      const uint32_t top = L - 1 - 3 * r;
-      nb = top + 1 >= 3 ? 3 : top + 1;
+      const uint32_t top = L - 1 - kRB * r;
+      nb = top + 1 >= kRB ? kRB : top + 1;
       lo_bit = top + 1 - nb;
     } else {
-      lo_bit = 3 * r;
-      nb = L - lo_bit >= 3 ? 3 : L - lo_bit;
+      lo_bit = kRB * r;
+      nb = L - lo_bit >= kRB ? kRB : L - lo_bit;
     }
     const uint32_t ptop = lo_bit + nb - 1;
-    switch (nb) {
-      case 3: run_round<3, FWD, MULV>(lds, g, first, last, ptop, L, Lg, jhi, lt, T, tw, active); break;
-      case 2: run_round<2, FWD, MULV>(lds, g, first, last, ptop, L, Lg, jhi, lt, T, tw, active); break;
-      default: run_round<1, FWD, MULV>(lds, g, first, last, ptop, L, Lg, jhi, lt, T, tw, active); break;
-    }
+    if (nb == kRB)
+      run_round<(int)kRB, FWD, MULV>(lds, g, first, last, ptop, L, Lg, jhi, lt, T, tw, active);
+    else if (kRB == 3 && nb == 2)
+      run_round<2, FWD, MULV>(lds, g, first, last, ptop, L, Lg, jhi, lt, T, tw, active);
+    else
+      run_round<1, FWD, MULV>(lds, g, first, last, ptop, L, Lg, jhi, lt, T, tw, active);
   }
 }
 
@@ -481,16 +488,22 @@ hipError_t set_lds(const void *kernel, size_t bytes) {
 
 namespace cfft_launch {
 
-// fft128 block held in one workgroup: 2048 points = 68 KiB of LDS, so two
-// workgroups share a CU (a 4096-point block, 136 KiB, leaves one per CU
-// waiting at every barrier; measured, batched n = 8192 forward 2.0 -> 2.7 M/s,
-// n = 16384 0.92 -> 1.19 M/s, n = 4096 forward 4.4 -> 5.2 M/s), except the
-// n = 4096 inverse, which keeps the whole transform in one block (5.2 against
-// 5.0 M/s).  Larger transforms (up to 2^kFft128MaxLog2) run their stages
-// above the block over global memory: forward first (CT runs from the top
-// bit down), inverse last (GS runs from the bottom bit up).
-constexpr uint32_t kFft128BlockLog2 = 11;
-constexpr uint32_t kFft128InvWholeLog2 = 12;
+// Points (log2) of the blocks held in a workgroup's LDS: 1024 (34 KiB, four per
+// CU), or 2048 (68 KiB, two) where that saves a pass over global memory and the
+// pass would cost more than waiting with fewer workgroups.  A transform of 2^Lg
+// points runs its stages above the block over global memory, three at a time:
+// forward first (CT runs from the top bit down), inverse last (GS runs from the
+// bottom bit up).  us on 2048- / 1024-point blocks, forward: n = 4096 26.5 / 20.6
+// (32 transforms), 101.9 / 91.0 (512); n = 8192 99.8 / 92.2 (256); n = 2048 19.6 /
+// 16.3 (1), 22.1 / 20.2 (64), 46.5 / 53.0 (512); n = 16384 25.6 / 21.6 (1), 29.4 /
+// 26.6 (8), 59.1 / 66.0 (64).  4096-point blocks (136 KiB) were slower throughout,
+// the whole n = 4096 inverse too at 32.6 and 89.4 against 16.4 and 87.5.
+constexpr uint64_t kFft128FewPoints = (uint64_t)1 << 17;
+uint32_t fft128_block_log2(uint32_t Lg, uint64_t batch) {
+  if (Lg <= 10) return Lg;
+  const uint32_t passes10 = (Lg - 10 + 2) / 3, passes11 = (Lg - 11 + 2) / 3;
+  return passes10 <= passes11 || (batch << Lg) <= kFft128FewPoints ? 10 : 11;
+}
 constexpr uint32_t kFft128MaxLog2 = 20;
 
 namespace {
@@ -531,7 +544,7 @@ hipError_t fft128_blocks(uint32_t L, uint32_t Lg, double *re0, double *re1, doub
   hipError_t e = set_lds(k, lds);
   if (e != hipSuccess) return e;
   const uint64_t wgs = (blocks + G - 1) / G;
-  hipLaunchKernelGGL((k_fft128<FWD, MULV>), dim3((uint32_t)wgs), dim3(G * (n / 8)), lds, s, re0,
+  hipLaunchKernelGGL((k_fft128<FWD, MULV>), dim3((uint32_t)wgs), dim3(G * (n >> kRB)), lds, s, re0,
                      re1, im0, im1, t_re0, t_re1, t_im0, t_im1, L, Lg, blocks);
   return hipGetLastError();
 }
@@ -540,9 +553,7 @@ template <bool FWD, int MULV>
 hipError_t fft128_any(uint32_t Lg, double *re0, double *re1, double *im0, double *im1,
                       const double *t_re0, const double *t_re1, const double *t_im0,
                       const double *t_im1, uint64_t batch, hipStream_t s) {
-  const uint32_t L = !FWD && Lg == kFft128InvWholeLog2 ? Lg
-                     : Lg < kFft128BlockLog2             ? Lg
-                                                         : kFft128BlockLog2;
+  const uint32_t L = fft128_block_log2(Lg, batch);
   hipError_t e = hipSuccess;
   if (FWD) {
     // bits Lg-1 .. L in rounds of up to 3 from the top, then the blocks

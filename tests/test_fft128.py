@@ -241,3 +241,33 @@ def test_gpu_plan_rejects_bad_sizes(cfft):
         cfft_amd.fft128.Plan(100)
     with pytest.raises(cfft_amd.CfftPanic):
         cfft_amd.fft128.Plan(1 << 21)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,batch", [(1024, 1), (2048, 64), (2048, 65), (4096, 3), (8192, 2),
+                                     (16384, 8), (16384, 9), (32768, 2), (131072, 2)])
+def test_gpu_block_sizes(cfft, O, n, batch):
+    """Blocks of 1024 or 2048 points by the number of global passes and, up to
+    2^17 points in all, by the batch (64 and 65 transforms of 2048, 8 and 9 of
+    16384): both directions bit-exact against the oracle on the first and
+    last transform, every transform the same for the same input."""
+    import cfft_amd
+    print("fft128 blocks: n=%d batch=%d" % (n, batch), flush=True)
+    rng = np.random.default_rng(n + batch)
+    z = rng.standard_normal((4, batch, n))
+    z[1] = z[0] * rng.uniform(-1, 1, (batch, n)) * 2.0**-54
+    z[3] = z[2] * rng.uniform(-1, 1, (batch, n)) * 2.0**-54
+    if batch > 2:
+        z[:, 1] = z[:, 0]
+    tw = O.fft128_twiddles(n)
+    dtw = dev(tw)
+    for f, ref in ((cfft_amd.fft128.negacyclic_fwd_fft, O.fft128_fwd),
+                   (cfft_amd.fft128.negacyclic_inv_fft, O.fft128_inv)):
+        d = dev(list(z))
+        f(*d, dtw, batch=batch)
+        got = np.stack([x.download() for x in d])
+        for b in sorted({0, batch - 1}):
+            want = np.stack(ref([z[i, b] for i in range(4)], tw))
+            assert np.array_equal(got[:, b], want), b
+        if batch > 2:
+            assert np.array_equal(got[:, 1], got[:, 0])
