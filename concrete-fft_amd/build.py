@@ -32,7 +32,7 @@ HIP_SOURCES = ["fft_kernels.hip", "polymul_kernels.hip", "polymul_n2048_kernels.
                "extprod_fused_kernels.hip", "uneven_kernels.hip", "noalloc.hip", "serve_kernels.hip",
                "large_transform_kernels.hip", "dit16_kernels.hip", "fixed_n256.hip", "fixed_n512.hip",
                "fixed_n1024.hip", "fixed_n2048.hip", "fixed_n4096.hip",
-               "fixed_n8192.hip"]
+               "fixed_n8192.hip", "fixed8_fft.hip"]
 HOST_HIP_SOURCES = ["api.cpp", "fft128_api.cpp", "products_api.cpp", "uneven_api.cpp",
                     "serve.cpp", "scratch.cpp", "host_stage.cpp"]
 GXX_SOURCES = ["host_tables.cpp", "twiddle128.cpp", "tune_cache.cpp"]

@@ -1,5 +1,6 @@
 """Mirror of `concrete_fft::fft128` (src/fft128/mod.rs) over the device C ABI."""
 import ctypes
+import math
 
 import numpy as np
 
@@ -26,7 +27,7 @@ class Plan:
         bufs = (re0, re1, im0, im1)
         if all(isinstance(x, DeviceBuffer) for x in bufs):
             if batch is None:
-                batch = int(np.prod(re0.shape)) // n
+                batch = math.prod(re0.shape) // n
             f = lib.cfft128_fwd if fwd else lib.cfft128_inv
             check(f(self.handle, re0.dptr, re1.dptr, im0.dptr, im1.dptr, batch,
                     stream.handle if stream else None))

@@ -6,6 +6,7 @@
 """
 import ctypes
 import enum
+import math
 
 import numpy as np
 
@@ -47,6 +48,7 @@ class Method:
 
 class _PlanBase:
     handle = None
+    _n = 0  # fft_size, kept after the first call
 
     def fft_size(self):
         n = ctypes.c_size_t(0)
@@ -65,9 +67,11 @@ class _PlanBase:
         return FftAlgo(a.value), b.value
 
     def _run(self, buf, fwd, stream=None, batch=None):
-        n = self.fft_size()
+        n = self._n if self.handle else 0
+        if not n:
+            n = self._n = self.fft_size()
         if isinstance(buf, DeviceBuffer):
-            total = int(np.prod(buf.shape))
+            total = math.prod(buf.shape)
             if buf.dtype != np.complex128:
                 raise TypeError("device buffer must be complex128")
             if batch is None:
@@ -84,7 +88,7 @@ class _PlanBase:
             raise CfftPanic(6, "assertion `left == right` failed\n  left: %d\n right: %d"
                             % (n, buf.shape[-1]))
         f = lib.cfft_fwd_host if fwd else lib.cfft_inv_host
-        check(f(self.handle, buf.ctypes.data, buf.size // n))
+        check(f(self.handle, buf.__array_interface__["data"][0], buf.size // n))
         return buf
 
     def fwd(self, buf, stream=None, batch=None):

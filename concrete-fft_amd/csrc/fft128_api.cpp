@@ -76,7 +76,7 @@ int run128_host(cfft_plan p, bool fwd, double *re0, double *re1, double *im0, do
         for (int i = 0; i < 4; ++i)
           std::memcpy(d + i * n * nb, h[i] + n * b0, n * nb * sizeof(double));
       },
-      [&](void *dv, size_t nb, hipStream_t s) {
+      [&](void *dv, size_t nb, hipStream_t s, cfft_launch::HostDone *) {
         double *d = static_cast<double *>(dv);
         return run128_plan(p, fwd, d, d + n * nb, d + 2 * n * nb, d + 3 * n * nb, nb, s);
       },

@@ -1,6 +1,7 @@
 // host_stage.cpp -- per-device pool of host staging slots (host_stage.hpp).
 #include "host_stage.hpp"
 
+#include <chrono>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -24,7 +25,7 @@ size_t slot_size(size_t bytes) {
 hipError_t grow(HostSlot *s, size_t bytes) {
   const size_t want = slot_size(bytes);
   if (s->pinned) {
-    // the slot's last call has synchronised its stream
+    // the slot's last call no longer uses it
     hipError_t e = hipHostFree(s->pinned);
     s->pinned = s->mapped = nullptr;
     s->bytes = 0;
@@ -45,7 +46,34 @@ hipError_t grow(HostSlot *s, size_t bytes) {
   return hipSuccess;
 }
 
+hipError_t make_flags(HostSlot *s) {
+  void *p = nullptr, *m = nullptr;
+  hipError_t e = hipHostMalloc(&p, kHostFlags * sizeof(uint32_t), hipHostMallocMapped);
+  if (e != hipSuccess) return e;
+  e = hipHostGetDevicePointer(&m, p, 0);
+  if (e != hipSuccess) {
+    (void)hipHostFree(p);
+    return e;
+  }
+  s->flags = static_cast<volatile uint32_t *>(p);
+  s->mapped_flags = static_cast<uint32_t *>(m);
+  return hipSuccess;
+}
+
 }  // namespace
+
+bool host_slot_poll(HostSlot *slot, uint32_t count) {
+  const auto give_up = std::chrono::steady_clock::now() + std::chrono::milliseconds(1);
+  for (uint32_t i = 0, spins = 0; i < count;) {
+    if (__atomic_load_n(&slot->flags[i], __ATOMIC_ACQUIRE) != 0) {
+      ++i;
+      continue;
+    }
+    if ((++spins & 1023u) == 0 && std::chrono::steady_clock::now() > give_up) return false;
+    __builtin_ia32_pause();
+  }
+  return true;
+}
 
 hipError_t host_slot_acquire(size_t bytes, HostSlot **out) {
   *out = nullptr;
@@ -70,6 +98,7 @@ hipError_t host_slot_acquire(size_t bytes, HostSlot **out) {
     slot->busy = true;
   }
   if (!slot->stream) e = hipStreamCreateWithFlags(&slot->stream, hipStreamNonBlocking);
+  if (e == hipSuccess && !slot->flags) e = make_flags(slot);
   if (e == hipSuccess && slot->bytes < bytes) e = grow(slot, bytes);
   if (e != hipSuccess) {
     host_slot_release(slot);

@@ -83,6 +83,20 @@ bool fixed_fft_n1024(const cfft_prog::Program &prog, dc64 *data, uint64_t ntrans
 bool fixed_fft_n2048(const cfft_prog::Program &prog, dc64 *data, uint64_t ntrans,
                      uint64_t stride, const dc64 *tw, hipStream_t s, hipError_t *e);
 
+// How a kernel tells a polling host that its results are written: each
+// workgroup sets its word of `flags` (mapped host memory, `capacity` words, all
+// zero before the launch) to 1; `used` is the number of words the launch will
+// set (0: it sets none, the stream has to be waited for).
+struct HostDone {
+  uint32_t *flags = nullptr;
+  uint32_t capacity = 0;
+  uint32_t used = 0;
+};
+// Whole transforms of 64 ... 1024 points for host calls (fixed8_fft.hpp); false, and nothing launched, for other programs or more
+// workgroups than `done` has words for.
+bool fft_fixed8(const cfft_prog::Program &prog, dc64 *data, uint64_t ntrans, uint64_t stride,
+                const dc64 *tw, HostDone *done, hipStream_t s, hipError_t *e);
+
 // Fused negacyclic product over the generic pass executor (a compile-time
 // program's kernel where one is built).
 hipError_t polymul_generic(const cfft_prog::Program &fwd, const cfft_prog::Program &inv,

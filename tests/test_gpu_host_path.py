@@ -83,3 +83,49 @@ def test_fft128_host_equals_device(cfft, n, batch):
         (plan.fwd if fwd else plan.inv)(*d)
         for a, b in zip(h, d):
             assert np.array_equal(a.view(np.uint64), b.download().view(np.uint64))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,batch", [(64, 1), (64, 7), (64, 512), (64, 513), (128, 5), (256, 3),
+                                     (512, 2), (1024, 1), (1024, 64), (1024, 65), (1024, 256),
+                                     (1024, 257), (8192, 3)])
+@pytest.mark.parametrize("algo", list(FftAlgo))
+def test_polled_host_calls_equal_device(cfft, n, batch, algo):
+    """Host calls of up to 4 MiB: groups of transforms partly filled, the most
+    workgroups that report to the polling host (64: 512 transforms of 64 points,
+    64 of 1024) and one transform more, the largest call on the pinned buffer
+    (256 transforms of 1024 points) and one through a device buffer; several
+    calls in a row on one slot; both directions."""
+    print("host path: polled n=%d batch=%d %s" % (n, batch, algo.name), flush=True)
+    plan = ordered.Plan(n, ordered.Method.UserProvided(algo), large=True)
+    rng = np.random.default_rng(n + batch)
+    for fwd in (True, False, True):
+        x = _rand(rng, batch, n)
+        h, d = _both(plan, x, fwd)
+        assert np.array_equal(h.view(np.uint64), d.view(np.uint64))
+
+
+@pytest.mark.gpu
+def test_polled_host_calls_from_threads(cfft):
+    """Threads sharing a plan each poll a slot of their own."""
+    import threading
+    print("host path: threads", flush=True)
+    plan = unordered.Plan(1024, unordered.Method.UserProvided(FftAlgo.Dif16, 512))
+    rng = np.random.default_rng(5)
+    xs = [_rand(rng, 3, 1024) for _ in range(4)]
+    want = [_both(plan, x, True)[1] for x in xs]
+    bad = []
+
+    def work(x, w):
+        for _ in range(50):
+            h = x.copy()
+            plan.fwd(h)
+            if not np.array_equal(h.view(np.uint64), w.view(np.uint64)):
+                bad.append(1)
+
+    ts = [threading.Thread(target=work, args=a) for a in zip(xs, want)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
