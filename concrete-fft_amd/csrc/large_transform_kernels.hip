@@ -306,6 +306,84 @@ k_depth8k_pair(c64 *__restrict__ data, uint64_t batch, uint64_t stride,
   }
 }
 
+// ---- the depth levels of a Dif16 / 1024 plan at n = 32768 in one pass over memory ----
+// Radix 8 at 32768 points, radix 4 in each 4096-point chunk (src/unordered.rs:
+// 391-489): thread jj holds the points jj + 1024 m, m < 32, which both levels
+// close over, so one pass reads and writes each point once and leaves (inverse:
+// takes) 1024-point chunks.  The first level's butterfly k2 < 4 takes m = 4 k + k2
+// and the second's kk < 8 the values m = 4 kk + k2 that the first left there.
+// HBM-bound (32 loads in flight per thread at 250 registers; at 168, three waves
+// per SIMD, it spills and took 170 us for 128).  Against a radix-8 pass and
+// 4096-point chunks, with the caller's copy in both: 256 transforms 131 -> 128 us
+// forward, 147 -> 138 inverse; 96 58.1 -> 52.7 and 61.3 -> 58.0.
+template <bool FWD>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 3)))
+k_depth32k_global(c64 *__restrict__ data, const c64 *__restrict__ tw) {
+  const uint64_t gid = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  const uint32_t jj = (uint32_t)gid & 1023u;
+  c64 *d = data + ((gid >> 10) << 15) + jj;
+  c64 v[32];
+#pragma unroll
+  for (uint32_t k2 = 0; k2 < 4; ++k2)
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) v[4 * k + k2] = d[1024 * (4 * k + k2)];
+  auto level8 = [&](uint32_t k2) {
+    c64 u[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int at = 4 * (FWD ? k : bitrev_digit<8>(k)) + (int)k2;
+      u[k] = v[at];
+      if (!FWD && k > 0) u[k] = cmul(conj(tw[(uint32_t)k * (jj + 1024 * k2)]), u[k]);
+    }
+    butterfly<8, FWD>(u);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int at = 4 * (FWD ? bitrev_digit<8>(k) : k) + (int)k2;
+      v[at] = FWD && k > 0 ? cmul(tw[(uint32_t)k * (jj + 1024 * k2)], u[k]) : u[k];
+    }
+  };
+  auto level4 = [&] {
+    c64 w[4];
+#pragma unroll
+    for (uint32_t k = 1; k < 4; ++k) {
+      w[k] = tw[(k * jj) << 3];
+      if (!FWD) w[k] = conj(w[k]);
+    }
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
+      c64 u[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        u[k] = v[4 * kk + (FWD ? k : bitrev_digit<4>(k))];
+        if (!FWD && k > 0) u[k] = cmul(w[k], u[k]);
+      }
+      butterfly<4, FWD>(u);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        v[4 * kk + (FWD ? bitrev_digit<4>(k) : k)] = FWD && k > 0 ? cmul(w[k], u[k]) : u[k];
+    }
+  };
+  if constexpr (FWD) {
+#pragma unroll
+    for (uint32_t k2 = 0; k2 < 4; ++k2) {
+      level8(k2);
+      sched_fence();
+    }
+    level4();
+#pragma unroll
+    for (uint32_t m = 0; m < 32; ++m) d[1024 * m] = v[m];
+  } else {
+    level4();
+#pragma unroll
+    for (uint32_t k2 = 0; k2 < 4; ++k2) {
+      level8(k2);
+#pragma unroll
+      for (uint32_t k = 0; k < 8; ++k) d[1024 * (4 * k + k2)] = v[4 * k + k2];
+      sched_fence();
+    }
+  }
+}
+
 }  // namespace
 
 namespace cfft_launch {
@@ -347,6 +425,19 @@ hipError_t depth8k_transform(bool fwd, dc64 *data, uint64_t batch, uint64_t stri
     hipLaunchKernelGGL(k_depth8k_pair<true>, grid, block, kLds, s, d, batch, stride, t, tb);
   else
     hipLaunchKernelGGL(k_depth8k_pair<false>, grid, block, kLds, s, d, batch, stride, t, tb);
+  return hipGetLastError();
+}
+
+// Dif16 plans with n = 32768 and base_n = 1024: both depth levels over a
+// contiguous batch (forward: before the 1024-point transforms, inverse: after
+// them); tw is the plan's 32768-point table.
+hipError_t depth32k_global(bool fwd, dc64 *data, uint64_t batch, const dc64 *tw, hipStream_t s) {
+  if (batch == 0) return hipSuccess;
+  c64 *d = reinterpret_cast<c64 *>(data);
+  const c64 *t = reinterpret_cast<const c64 *>(tw);
+  const dim3 grid((uint32_t)(batch * 4));  // 1024 threads per transform
+  if (fwd) hipLaunchKernelGGL(k_depth32k_global<true>, grid, dim3(256), 0, s, d, t);
+  else hipLaunchKernelGGL(k_depth32k_global<false>, grid, dim3(256), 0, s, d, t);
   return hipGetLastError();
 }
 

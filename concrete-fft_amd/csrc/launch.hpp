@@ -163,6 +163,9 @@ hipError_t w2048_transform(bool fwd, dc64 *data, uint64_t batch, uint64_t stride
 hipError_t depth16k_transform(bool fwd, dc64 *data, uint64_t batch, uint64_t stride,
                               const dc64 *tw, const dc64 *tw2, const dc64 *tw_blk,
                               hipStream_t s);
+// Dif16 plans with n = 32768 and base_n = 1024: the plan's two depth levels over
+// a contiguous batch, in one pass over memory (tw: the plan's table).
+hipError_t depth32k_global(bool fwd, dc64 *data, uint64_t batch, const dc64 *tw, hipStream_t s);
 // Dif16 plans with n = 8192 and base_n = 1024: the plan's radix-8 depth level
 // in registers, two transforms per workgroup through LDS in turn.
 hipError_t depth8k_transform(bool fwd, dc64 *data, uint64_t batch, uint64_t stride,

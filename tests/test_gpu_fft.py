@@ -329,3 +329,26 @@ def test_dit16_register_form(cfft, oracle, batch, stride):
     w = d.download()
     assert np.array_equal(w[:, :n], oracle.unordered_inv(ref, 7, 1024))
     assert np.array_equal(w[:, n:], x[:, n:])
+
+
+@pytest.mark.parametrize("batch", [63, 64, 67])
+def test_n32768_depth_levels_in_one_pass(cfft, oracle, batch):
+    """n = 32768 on Dif16 / 1024: a batch of 64 takes both depth levels in one
+    pass over memory, one of 63 (or a strided one) the levels by themselves;
+    every transform equals the oracle's or its own call's."""
+    from cfft_amd.device import DeviceBuffer
+    from cfft_amd.unordered import FftAlgo, Method, Plan
+    print("n=32768 batch=%d" % batch, flush=True)
+    n = 32768
+    rng = np.random.default_rng(batch)
+    x = rand_c(rng, (batch, n))
+    plan = Plan(n, Method.UserProvided(FftAlgo.Dif16, 1024))
+    for run, ref in ((plan.fwd, oracle.unordered_fwd), (plan.inv, oracle.unordered_inv)):
+        d = DeviceBuffer.from_host(x)
+        run(d)
+        got = d.download()
+        for b in (0, batch // 2, batch - 1):
+            assert np.array_equal(got[b], ref(x[b], 6, 1024)), b
+        one = DeviceBuffer.from_host(x[1:2])
+        run(one)
+        assert np.array_equal(one.download()[0], got[1])
