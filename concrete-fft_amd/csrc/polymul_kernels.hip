@@ -319,9 +319,16 @@ __device__ __forceinline__ void depth_raw_to_lds(const DepthRaw<LOG2N> &d, c64 *
 // Persistent form: each workgroup loops over its share of the batch, G
 // products at a time.  PRE_B: B's inputs are loaded while A's base transform
 // runs; PRE_A: the next round's A inputs are loaded while the inverse base
-// transform runs (so only the first round waits for A).  A group past the
-// batch works on the workgroup's first product of that round and stores
-// nothing; every wave runs every round and reaches every barrier.
+// transform runs (so only the first round waits for A).  Group g's products
+// are g * grid + block + round * G * grid: consecutive products go to
+// different workgroups, so a last round that does not fill the chip (or a
+// batch below G per CU) is spread over the CUs, one product on each, where
+// two or four of them on part of the CUs had left the others idle (N = 4096:
+// 600 products 26.4 -> 23.3 us, 1100 47.2 -> 39.3; N = 8192: 600 48.8 -> 43.3;
+// batches that fill every round the same within 1 %).  A group whose share is
+// done ends; a barrier waits on the waves that are left.  A barrier of each
+// product's own (a counter in LDS) instead of the workgroup's was slower:
+// 33.3 against 30.1 us for 512 products of N = 8192.
 template <int LOG2N, bool PRE_B, bool PRE_A>
 __global__ void __launch_bounds__(64 * kPW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_depth_polymul(const uint64_t *__restrict__ A, const int64_t *__restrict__ B,
@@ -338,26 +345,26 @@ k_depth_polymul(const uint64_t *__restrict__ A, const int64_t *__restrict__ B,
   extern __shared__ c64 smem[];
   c64 *ltw = smem;
   for (uint32_t i = threadIdx.x; i < kTwWords; i += blockDim.x) ltw[i] = tw_blk[i];
+  const uint32_t grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / TJ);
   const uint64_t step = (uint64_t)gridDim.x * G;
-  // round r of this workgroup: products blockIdx.x * G + r * step + g
-  auto offset_of = [&](uint64_t first, uint32_t g) -> uint64_t {
-    const uint64_t pr = first + g;
-    return (pr < batch ? pr : first) * (2ull * n);
+  // a group past the batch (or without a next round) loads from the twist
+  // table, 2 n words that the L2 holds, and never uses what it got
+  auto words_of = [&](uint64_t p) {
+    return p < batch ? A + p * (2ull * n) : reinterpret_cast<const uint64_t *>(twist);
   };
-  uint64_t first = (uint64_t)blockIdx.x * G;
+  uint64_t p = (uint64_t)grp * gridDim.x + blockIdx.x;
   DepthRaw<LOG2N> ra;
-  if (PRE_A) depth_raw_load<LOG2N>(ra, A + offset_of(first, threadIdx.x / TJ), threadIdx.x % TJ);
+  if (PRE_A) depth_raw_load<LOG2N>(ra, words_of(p), threadIdx.x % TJ);
   __syncthreads();  // twiddle block staged
-  while (first < batch) {
+  while (p < batch) {
     // recomputed per round (opaque) so the per-lane addresses below are not
     // hoisted out of the loop and kept live across it
     const uint32_t tid = launder_u32(threadIdx.x);
-    const uint32_t g = tid / TJ, t = tid % TJ;
-    c64 *X = smem + kTwWords + g * (R * CH);
+    const uint32_t t = tid % TJ;
+    c64 *X = smem + kTwWords + grp * (R * CH);
     const uint32_t c = t >> 6, l = t & 63;
     c64 *xc = X + c * CH;
-    const bool active = first + g < batch;
-    const uint64_t off = offset_of(first, g);
+    const uint64_t off = p * (2ull * n);
     if (!PRE_A) depth_raw_load<LOG2N>(ra, A + off, t);
     depth_raw_to_lds<LOG2N, true>(ra, X, t, tw, twist);
     __syncthreads();
@@ -384,10 +391,9 @@ k_depth_polymul(const uint64_t *__restrict__ A, const int64_t *__restrict__ B,
 #pragma unroll
       for (uint32_t s = 0; s < 16; ++s) fa[s] = cmul(fa[s], fb[s]);
     }
-    const uint64_t next = first + step;
+    const uint64_t next = p + step;
     if (PRE_A) {
-      // the next round's A (past the batch: this round's, never used)
-      depth_raw_load<LOG2N>(ra, A + offset_of(next < batch ? next : first, g), t);
+      depth_raw_load<LOG2N>(ra, words_of(next), t);  // the next round's A
       sched_fence();
     }
     c64 u[16];
@@ -411,18 +417,16 @@ k_depth_polymul(const uint64_t *__restrict__ A, const int64_t *__restrict__ B,
         w[k] = cmul(f, w[k]);
       }
       butterfly<R, false>(w);
-      if (active) {
 #pragma unroll
-        for (int k = 0; k < R; ++k) {
-          const uint32_t q = (uint32_t)k * 1024 + j;
-          const c64 r = cmul(untwist[q], w[k]);
-          st_stream(from_torus(r.re), &cp[q]);
-          st_stream(from_torus(r.im), &cp[q + n]);
-        }
+      for (int k = 0; k < R; ++k) {
+        const uint32_t q = (uint32_t)k * 1024 + j;
+        const c64 r = cmul(untwist[q], w[k]);
+        st_stream(from_torus(r.re), &cp[q]);
+        st_stream(from_torus(r.im), &cp[q + n]);
       }
     }
     __syncthreads();  // every chunk read before the next round's depth pass
-    first = next;
+    p = next;
   }
 }
 
@@ -976,9 +980,7 @@ hipError_t depth_polymul(uint32_t log2n, const uint64_t *a, const int64_t *b, ui
   if (e != hipSuccess) return e;
   const c64 *t = reinterpret_cast<const c64 *>(tw), *tb = reinterpret_cast<const c64 *>(tw_blk);
   const c64 *z = reinterpret_cast<const c64 *>(twist), *u = reinterpret_cast<const c64 *>(untwist);
-  const uint64_t per_wg = 8u >> (log2n - 10);  // 8 / R products per round
-  const uint64_t want = (batch + per_wg - 1) / per_wg;
-  const dim3 grid((uint32_t)(want < (uint64_t)cus ? want : (uint64_t)cus)), block(64 * kPW);
+  const dim3 grid((uint32_t)(batch < (uint64_t)cus ? batch : (uint64_t)cus)), block(64 * kPW);
   if (log2n == 11)
     hipLaunchKernelGGL((k_depth_polymul<11, true, true>), grid, block, lds, s, a, b, c, batch, t,
                        tb, z, u);

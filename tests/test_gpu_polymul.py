@@ -261,3 +261,22 @@ def test_dif16_product_routes_meet(cfft, oracle, N, base_n):
     for batch in (last, last + 1):
         c = products.negacyclic_polymul_u64_host(plan, a[:batch], b[:batch])
         assert np.array_equal(c, ref[:batch]), batch
+
+
+@pytest.mark.parametrize("N,batch", [(4096, 513), (4096, 1024), (4096, 1281), (8192, 257),
+                                     (8192, 511), (8192, 770), (16384, 129), (16384, 259)])
+def test_depth_product_rounds(cfft, oracle, N, batch):
+    """Register-resident products with a depth pass: batches that end inside
+    a round, one group of a workgroup after another; every product equals the
+    eight-point kernel's (small batches) and the oracle's at both ends."""
+    from cfft_amd import products
+    from cfft_amd.unordered import FftAlgo, Method, Plan
+    print("N=%d batch=%d" % (N, batch), flush=True)
+    plan = Plan(N // 2, Method.UserProvided(FftAlgo.Dif16, 1024))
+    a, b = rand_inputs(N + batch, batch, N)
+    got = products.negacyclic_polymul_u64_host(plan, a, b)
+    for i in range(0, batch, 128):
+        assert np.array_equal(products.negacyclic_polymul_u64_host(
+            plan, a[i:i + 128], b[i:i + 128]), got[i:i + 128]), i
+    for i in (0, batch - 1):
+        assert np.array_equal(oracle.polymul_f64(a[i:i + 1], b[i:i + 1], 6, 1024)[0], got[i])
