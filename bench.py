@@ -57,16 +57,16 @@ PEAK_HBM_GBS = 8000.0
 PEAK_FP64_TFLOPS = 78.6  # MI355X dense FP64 (vector and matrix)
 BYTES_PER_PRODUCT = 24 * N  # A 8N + B 8N read, C 8N written
 # HBM bytes per 8192-product launch of the persistent Dif16 kernel, from
-# rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE over 4 launches: FETCH_SIZE x 2
+# rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE over 3 launches: FETCH_SIZE x 2
 # (the counter reads half of a plain copy kernel's known read size on this
-# platform) + WRITE_SIZE (exact for a copy): (131391 x 2 + 131113) KiB.  The
+# platform) + WRITE_SIZE (exact for a copy): (131384 x 2 + 131114) KiB.  The
 # figure holds for the kernel sources it was measured on (their SHA-256
 # below); when they change, `traffic` is reported as null until the counters
 # are run again.
-TRAFFIC_BYTES = (131391 * 2 + 131113) * 1024
+TRAFFIC_BYTES = (131384 * 2 + 131114) * 1024
 TRAFFIC_SOURCES = ("concrete-fft_amd/csrc/polymul_n2048_kernels.hip", "concrete-fft_amd/csrc/r16_exec.hpp",
                    "concrete-fft_amd/csrc/device_math.hpp")
-TRAFFIC_SHA256 = "ac50f118ad451f083dbf608844c3896354b4151d9029465d44a98b7a9a635fa4"
+TRAFFIC_SHA256 = "4782eec616e719e2ad981a208033936b6ac7871c8d24e12f5ca69145d364fcc9"
 
 
 def traffic_sources_sha():

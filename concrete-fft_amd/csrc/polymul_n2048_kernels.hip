@@ -63,7 +63,10 @@ k_r16_polymul_persistent(const uint64_t *__restrict__ A, const int64_t *__restri
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   c64 *x = smem + kPmHead + wave * kPmX;
   const uint64_t step = (uint64_t)gridDim.x * kPW;
-  uint64_t poly = (uint64_t)blockIdx.x * kPW + wave;
+  // dealt over the workgroups one by one: a round that does not fill the chip
+  // leaves no CU idle (1100 products 20.7 -> 18.5 us, 3000 37.7 -> 29.9; full
+  // rounds the same)
+  uint64_t poly = (uint64_t)wave * gridDim.x + blockIdx.x;
   uint64_t pb[32];  // raw words of B for the wave's current product
   if (poly < batch) {
     const uint32_t l = threadIdx.x & 63u;
@@ -150,8 +153,7 @@ hipError_t launch_polymul_persistent(const uint64_t *a, const int64_t *b, uint64
       cus = it->second;
     }
   }
-  const uint64_t want = (batch + kPW - 1) / kPW;
-  const uint32_t grid = (uint32_t)(want < (uint64_t)cus ? want : (uint64_t)cus);
+  const uint32_t grid = (uint32_t)(batch < (uint64_t)cus ? batch : (uint64_t)cus);
   hipLaunchKernelGGL(k_r16_polymul_persistent, dim3(grid), dim3(64 * kPW), kPersistLds, s, a, b,
                      c, batch, reinterpret_cast<const c64 *>(tw), reinterpret_cast<const c64 *>(twist));
   return hipGetLastError();

@@ -352,3 +352,26 @@ def test_n32768_depth_levels_in_one_pass(cfft, oracle, batch):
         one = DeviceBuffer.from_host(x[1:2])
         run(one)
         assert np.array_equal(one.download()[0], got[1])
+
+
+@pytest.mark.parametrize("n,base_n", [(512, 512), (1024, 512), (1024, 1024), (2048, 1024)])
+def test_wave_transforms_dealt(cfft, oracle, n, base_n):
+    """Wave-local transforms are dealt over the workgroups in grids of up to
+    512: batches below one wave per CU, at a ragged end, inside the second
+    window of 256 workgroups and past 512, forward and back."""
+    from cfft_amd.device import DeviceBuffer
+    from cfft_amd.unordered import FftAlgo, Method, Plan
+    per_wg = 8 * {(512, 512): 4, (1024, 512): 2, (1024, 1024): 2, (2048, 1024): 1}[(n, base_n)]
+    plan = Plan(n, Method.UserProvided(FftAlgo.Dif16, base_n))
+    rng = np.random.default_rng(n + base_n)
+    x = rand_c(rng, (512 * per_wg + 1, n))
+    for batch in (1, 257, 256 * per_wg + 3, 512 * per_wg, 512 * per_wg + 1):
+        print("n=%d base=%d batch=%d" % (n, base_n, batch), flush=True)
+        d = DeviceBuffer.from_host(x[:batch])
+        plan.fwd(d)
+        got = d.download()
+        for b in sorted({0, batch // 2, batch - 2, batch - 1} - {-1}):
+            assert np.array_equal(got[b], oracle.unordered_fwd(x[b], 6, base_n)), (batch, b)
+        plan.inv(d)
+        back = d.download()
+        assert np.max(np.abs(back / n - x[:batch])) < 1e-13

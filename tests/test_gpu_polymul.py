@@ -280,3 +280,19 @@ def test_depth_product_rounds(cfft, oracle, N, batch):
             plan, a[i:i + 128], b[i:i + 128]), got[i:i + 128]), i
     for i in (0, batch - 1):
         assert np.array_equal(oracle.polymul_f64(a[i:i + 1], b[i:i + 1], 6, 1024)[0], got[i])
+
+
+@pytest.mark.parametrize("N,base_n,batch", [(512, 256, 4097), (512, 256, 8197), (1024, 512, 2049),
+                                            (1024, 512, 4099), (2048, 1024, 1025),
+                                            (2048, 1024, 2051), (2048, 512, 1025),
+                                            (2048, 512, 2051)])
+def test_wave_products_dealt(cfft, oracle, N, base_n, batch):
+    """Wave-local products are dealt over the workgroups: batches that end
+    inside a round, with a ragged last wave, give the oracle's words."""
+    from cfft_amd import products
+    from cfft_amd.unordered import FftAlgo, Method, Plan
+    print("N=%d base=%d batch=%d" % (N, base_n, batch), flush=True)
+    plan = Plan(N // 2, Method.UserProvided(FftAlgo.Dif16, base_n))
+    a, b = rand_inputs(N + batch, batch, N)
+    got = products.negacyclic_polymul_u64_host(plan, a, b)
+    assert np.array_equal(got, oracle.polymul_f64(a, b, 6, base_n))
