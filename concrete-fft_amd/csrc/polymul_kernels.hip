@@ -363,23 +363,28 @@ k_depth_polymul(const uint64_t *__restrict__ A, const int64_t *__restrict__ B,
   const uint32_t grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / TJ);
   const uint64_t step = (uint64_t)gridDim.x * G;
   // a group past the batch (or without a next round) loads from the twist
-  // table, 2 n words that the L2 holds, and never uses what it got
-  auto words_of = [&](uint64_t p) {
+  // table, 2 n words that the L2 holds, and never uses what it got (777 of
+  // N = 8192: 50.2 us against 52.9 with its own A again); at G = 1 its own A
+  auto words_of = [&](uint64_t p, uint32_t g) {
+    if (G == 1) return A + ((p < batch ? p : blockIdx.x) + g) * (2ull * n);
     return p < batch ? A + p * (2ull * n) : reinterpret_cast<const uint64_t *>(twist);
   };
   uint64_t p = (uint64_t)grp * gridDim.x + blockIdx.x;
   DepthRaw<LOG2N> ra;
-  if (PRE_A) depth_raw_load<LOG2N>(ra, words_of(p), threadIdx.x % TJ);
+  if (PRE_A) depth_raw_load<LOG2N>(ra, words_of(p, threadIdx.x / TJ), threadIdx.x % TJ);
   __syncthreads();  // twiddle block staged
   while (p < batch) {
     // recomputed per round (opaque) so the per-lane addresses below are not
     // hoisted out of the loop and kept live across it
     const uint32_t tid = launder_u32(threadIdx.x);
-    const uint32_t t = tid % TJ;
-    c64 *X = smem + kTwWords + grp * (R * CH);
+    // (at G = 1, where the group is 0, it stays a per-lane value, which keeps
+    // the addresses in vector registers: scalar ones cost 2 % at N = 16384)
+    const uint32_t g = G == 1 ? tid / TJ : grp, t = tid % TJ;
+    c64 *X = smem + kTwWords + g * (R * CH);
     const uint32_t c = t >> 6, l = t & 63;
     c64 *xc = X + c * CH;
-    const uint64_t off = p * (2ull * n);
+    const bool active = G > 1 || p + g < batch;
+    const uint64_t off = (G == 1 ? p + g : p) * (2ull * n);
     if (!PRE_A) depth_raw_load<LOG2N>(ra, A + off, t);
     depth_raw_to_lds<LOG2N, true>(ra, X, t, tw, twist);
     __syncthreads();
@@ -408,7 +413,8 @@ k_depth_polymul(const uint64_t *__restrict__ A, const int64_t *__restrict__ B,
     }
     const uint64_t next = p + step;
     if (PRE_A) {
-      depth_raw_load<LOG2N>(ra, words_of(next), t);  // the next round's A
+      // the next round's A
+      depth_raw_load<LOG2N>(ra, words_of(next < batch || G > 1 ? next : p, g), t);
       sched_fence();
     }
     c64 u[16];
@@ -432,12 +438,14 @@ k_depth_polymul(const uint64_t *__restrict__ A, const int64_t *__restrict__ B,
         w[k] = cmul(f, w[k]);
       }
       butterfly<R, false>(w);
+      if (active) {
 #pragma unroll
-      for (int k = 0; k < R; ++k) {
-        const uint32_t q = (uint32_t)k * 1024 + j;
-        const c64 r = cmul(untwist[q], w[k]);
-        st_stream(from_torus(r.re), &cp[q]);
-        st_stream(from_torus(r.im), &cp[q + n]);
+        for (int k = 0; k < R; ++k) {
+          const uint32_t q = (uint32_t)k * 1024 + j;
+          const c64 r = cmul(untwist[q], w[k]);
+          st_stream(from_torus(r.re), &cp[q]);
+          st_stream(from_torus(r.im), &cp[q + n]);
+        }
       }
     }
     __syncthreads();  // every chunk read before the next round's depth pass
