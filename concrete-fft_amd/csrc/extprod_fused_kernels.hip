@@ -30,6 +30,7 @@
 
 #include <type_traits>
 
+#include "extprod_rows.hpp"
 #include "gadget.hpp"
 #include "launch.hpp"
 #include "lds_attr.hpp"
@@ -74,8 +75,8 @@ __device__ __forceinline__ c64 twist_point(const c64 *ltz, uint32_t ch, uint32_t
 }
 
 // A buffer descriptor over `points` points: loads take a 32-bit offset per lane
-// and a scalar one (which the bounds check leaves out), and return zeros past
-// the end without reading memory.
+// and a scalar one in place of a 64-bit address.  Every load stays inside the
+// `points`.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t point_buffer(const c64 *base, uint32_t points) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<c64 *>(base), 0, (int)(points * 16u),
                                            0x00027000);
@@ -101,7 +102,7 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
   using F = FGeom<LOG2N>;
   using S = R16<F::LB>;
   constexpr uint32_t n = F::n, T = F::T, CH = F::CH;
-  constexpr uint32_t RG = F::U / CH / P;  // rows of one GLWE in a round
+  constexpr uint32_t RG = rows_per_round(F::U, CH, P);
   static_assert(RG >= 1 && P * K1 * CH <= F::U, "the columns must fit the units");
   extern __shared__ c64 smem[];
   c64 *ltw = smem, *ltz = smem + kSTw, *xs = smem + F::head;
@@ -145,9 +146,10 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
     const auto blk = point_buffer(tw_blk, 16 * 64 + 16 * 4), zt = point_buffer(twist, n);
     auto entry = [&](uint32_t i) { return load_point(blk, r16s_block_index(i)); };
     const c64 t0 = entry(tid), t1 = entry(tid + 512);
-    // (n = 512: one twist entry per thread; n = 2048: entry 1024 as well)
-    const c64 z0 = load_point(zt, tid), z1 = load_point(zt, F::zw > 512 ? tid + 512 : n);
-    const c64 z2 = load_point(zt, F::zw > 1024 ? 1024 : n);
+    // (n = 512: one twist entry per thread; n = 2048: entry 1024 as well; entry 0
+    // where there is none)
+    const c64 z0 = load_point(zt, tid), z1 = load_point(zt, F::zw > 512 ? tid + 512 : 0);
+    const c64 z2 = load_point(zt, F::zw > 1024 ? 1024 : 0);
     fetch(g0, 0);
     sched_fence();
     ltw[tid] = t0;
@@ -227,13 +229,11 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
       // the first ones before the transform that hides them where they fit
       // beside it and the sums (spilling cost more)
       constexpr uint32_t PT = CH * F::PB;
-      constexpr uint32_t KM = (CH == 1 ? 24 : 16) / (PT * K1);
-      constexpr uint32_t K8 = KM < 1 ? 1 : KM < 8 ? KM : 8, KR = K8 < RG ? K8 : RG;
+      constexpr uint32_t KR = rows_requested(CH, PT, K1, RG);
       constexpr bool EARLY = CH == 1 && P <= 2 && 4 * (P + KR) * PT * K1 <= 120;
       const uint32_t nr = rows - r0 < RG ? rows - r0 : RG;
       c64 kv[KR][PT][K1];
       auto key_rows = [&](uint32_t rr) {
-        // (a row past the round's last is an empty buffer: no memory read)
         const uint32_t t = launder_u32(tid);
         uint32_t q[PT];
 #pragma unroll
@@ -243,8 +243,8 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
         }
 #pragma unroll
         for (uint32_t i = 0; i < KR; ++i) {
-          const auto key = point_buffer(keyf + (uint64_t)(r0 + rr + i) * (K1 * n),
-                                        rr + i < nr ? K1 * n : 0);
+          const auto key = point_buffer(keyf + (uint64_t)key_row(r0, rr, i, rows) * (K1 * n),
+                                        K1 * n);
 #pragma unroll
           for (uint32_t e = 0; e < PT; ++e)
 #pragma unroll
