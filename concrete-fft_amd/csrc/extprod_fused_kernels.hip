@@ -230,7 +230,15 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
       // beside it and the sums (spilling cost more)
       constexpr uint32_t PT = CH * F::PB;
       constexpr uint32_t KR = rows_requested(CH, PT, K1, RG);
-      constexpr bool EARLY = CH == 1 && P <= 2 && 4 * (P + KR) * PT * K1 <= 120;
+      // and the next coefficients before the sums where they fit beside the key
+      // points, after them elsewhere.  Requested before them by every form, 64-bit
+      // words spilled 28-196 bytes per lane at k1 = 3 and 4, 32-bit ones 68 at N =
+      // 2048, k1 = 4, P = 2 (us, so and now, N = 2048: k1 = 3, 1 level of 32 bits,
+      // 600 GLWEs 46.2 / 37.0; 4 levels of 10, 1100 162.9 / 110.7; k1 = 4, 8 levels
+      // of 8, 257 160.9 / 101.5; 3 levels of 8, 600 113.4 / 83.6).
+      constexpr uint32_t KREGS = 4 * (P + KR) * PT * K1;  // key points and sums
+      constexpr bool EARLY = CH == 1 && P <= 2 && KREGS <= 120;
+      constexpr bool AHEAD = NARROW ? KREGS <= 144 : CH == 1 && KREGS <= (PT == 1 ? 108 : 112);
       const uint32_t nr = rows - r0 < RG ? rows - r0 : RG;
       c64 kv[KR][PT][K1];
       auto key_rows = [&](uint32_t rr) {
@@ -268,7 +276,7 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
       auto fetch_next = [&]() {
         fetch(more ? g0 : g0 + (uint64_t)gridDim.x * P, more ? r0 + RG : 0);
       };
-      if constexpr (CH == 1 || NARROW) fetch_next();
+      if constexpr (AHEAD) fetch_next();
       sched_fence();
       __syncthreads();
       const uint32_t t = launder_u32(tid);
@@ -291,9 +299,9 @@ k_extprod_fused(const c64 *__restrict__ keyf, const uint64_t *glwe, const uint64
           }
         }
       }
-      if constexpr (CH == 2 && !NARROW) {
+      if constexpr (!AHEAD) {
         sched_fence();
-        fetch_next();  // (64-bit words would spill beside the key points)
+        fetch_next();
       }
       __syncthreads();  // every spectrum of the round read
     }

@@ -149,6 +149,10 @@ def test_large_batch_runs_in_passes(cfft, oracle):
     (1024, 2, 3, 8, 1), (1024, 3, 2, 10, 257), (1024, 2, 1, 23, 1029), (1024, 4, 5, 6, 515),
     (2048, 2, 3, 8, 1), (2048, 4, 5, 6, 258), (2048, 2, 3, 8, 1027), (2048, 3, 2, 16, 513),
     (4096, 2, 2, 15, 1), (4096, 3, 1, 23, 259), (4096, 2, 3, 8, 515), (4096, 4, 3, 8, 2),
+    # the widest digits of 32-bit words (levels * base_log = 31) and 64-bit words
+    (1024, 2, 1, 31, 513), (1024, 3, 2, 32, 600), (1024, 4, 5, 7, 515), (2048, 2, 1, 31, 257),
+    (2048, 3, 4, 16, 515), (2048, 4, 2, 32, 515), (4096, 2, 1, 31, 515), (4096, 2, 2, 16, 515),
+    (4096, 2, 2, 32, 259), (4096, 3, 4, 10, 400), (4096, 4, 1, 32, 259),
 ])
 def test_fused_product_groups(cfft, oracle, N, k1, levels, base_log, batch):
     """The one-launch form (k1 = 2 ... 4): 1, 2 or 4 GLWEs per workgroup
