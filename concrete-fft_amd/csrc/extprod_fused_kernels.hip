@@ -443,22 +443,6 @@ hipError_t launch_fused_k(const FArgs &a, uint32_t k1, hipStream_t s) {
 
 namespace cfft_launch {
 
-// The one-launch form takes k1 = 2 ... 4 (its column sums are registers).  It
-// measured 1.1x to 2.7x faster than the split form over N = 1024, 2048, 4096,
-// 2 to 12 rows and 1 to 2000 GLWEs.  With many rows and few GLWEs one CU runs
-// in rounds the rows that the split form spreads over idle CUs: from 4 rounds
-// on the split form is ahead below about 2 rounds^2 GLWEs (us, split against
-// fused: N = 4096, 16 rows, 4 rounds: 51.9 / 60.2 for 8 GLWEs, 64.0 / 61.1 for
-// 40; 32 rows, 8 rounds: 100 / 126 for 64, 288 / 251 for 260; N = 2048, 32
-// rows: 52.0 / 56.8 for 24, 57.7 / 57.0 for 40).
-bool external_product_fused_supported(uint32_t log2n, uint64_t batch, uint32_t k1,
-                                      uint32_t levels) {
-  if (log2n < 9 || log2n > 11 || k1 < 2 || k1 > 4) return false;
-  const uint32_t rows_per_round = log2n == 9 ? 16 : log2n == 10 ? 8 : 4;
-  const uint64_t rounds = (k1 * levels + rows_per_round - 1) / rows_per_round;
-  return rounds < 4 || batch >= 2 * rounds * rounds;
-}
-
 hipError_t external_product_fused(uint32_t log2n, const dc64 *keyf, const uint64_t *glwe,
                                   const uint64_t *glwe_tab, uint64_t *out,
                                   const uint64_t *out_tab, uint64_t batch, uint32_t k1,

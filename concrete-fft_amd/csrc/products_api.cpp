@@ -6,7 +6,9 @@
 #include <string>
 
 #include "cfft.h"
+#include "extprod_rows.hpp"
 #include "launch.hpp"
+#include "lds_attr.hpp"
 #include "plan.hpp"
 #include "scratch.hpp"
 
@@ -37,8 +39,6 @@ hipError_t external_product_split_w(uint32_t log2n, const dc64 *keyf, const uint
                                     uint32_t levels, uint32_t base_log, const dc64 *tw,
                                     const dc64 *tw_blk, const dc64 *twist, const dc64 *untwist,
                                     dc64 *scratch, hipStream_t s);
-bool external_product_fused_supported(uint32_t log2n, uint64_t batch, uint32_t k1,
-                                      uint32_t levels);
 hipError_t external_product_fused(uint32_t log2n, const dc64 *keyf, const uint64_t *glwe,
                                   const uint64_t *glwe_tab, uint64_t *out,
                                   const uint64_t *out_tab, uint64_t batch, uint32_t k1,
@@ -140,9 +140,13 @@ int external_product_with_scratch(cfft_plan plan, const void *key_fourier, int k
   // split form, which reads a whole pass before it writes.
   const size_t span = batch * glwe_words;
   const bool shifted = glwe && out && glwe != out && glwe < out + span && out < glwe + span;
-  if (blk && !shifted && (plan->n < 2048 || plan->twist_mirrored) &&
-      cfft_launch::external_product_fused_supported(ilog2(plan->n), batch, (uint32_t)k1,
-                                                    (uint32_t)levels))
+  int cus = 0;
+  if (blk && !shifted && (plan->n < 2048 || plan->twist_mirrored)) {
+    e = cfft_launch::cu_count(&cus);
+    if (e != hipSuccess) return hip_error(e, "external product");
+  }
+  if (cus > 0 && cfft_dev::one_launch(ilog2(plan->n), batch, (uint32_t)k1, (uint32_t)levels,
+                                      (uint32_t)base_log, (uint32_t)cus))
     return hip_error(cfft_launch::external_product_fused(
                          ilog2(plan->n), reinterpret_cast<const cfft_launch::dc64 *>(key_fourier),
                          glwe, glwe_tab, out, out_tab, batch, (uint32_t)k1, (uint32_t)levels,

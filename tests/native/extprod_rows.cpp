@@ -1,11 +1,23 @@
-// Key rows requested by the one-launch external product, one line per request:
-// log2n k1 glwes levels r0 rr i rows requested_row
+// Without arguments: the key rows requested by the one-launch external product,
+// one line per request: log2n k1 glwes levels r0 rr i rows requested_row.
+// With an argument: for every line "N k1 levels base_log batch cus" of the
+// input, 1 if the call runs on that form, else 0.
 #include <cstdint>
 #include <cstdio>
 
 #include "extprod_rows.hpp"
 
-int main() {
+int main(int argc, char **) {
+  if (argc > 1) {
+    unsigned N, k1, levels, base_log, cus;
+    unsigned long long batch;
+    while (std::scanf("%u %u %u %u %llu %u", &N, &k1, &levels, &base_log, &batch, &cus) == 6) {
+      uint32_t log2n = 0;
+      while ((2u << log2n) < N) ++log2n;
+      std::printf("%d\n", cfft_dev::one_launch(log2n, batch, k1, levels, base_log, cus) ? 1 : 0);
+    }
+    return 0;
+  }
   for (uint32_t log2n = 9; log2n <= 11; ++log2n)
     for (uint32_t k1 = 2; k1 <= 4; ++k1)
       for (uint32_t glwes = 1; glwes <= 4; glwes *= 2)
