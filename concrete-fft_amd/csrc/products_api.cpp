@@ -77,6 +77,12 @@ uint32_t ilog2(size_t n) {
   while (((size_t)1 << l) < n) ++l;
   return l;
 }
+// Whether two buffers of `words` words overlap other than exactly.  The
+// one-launch forms write an item's result while later items are still to be
+// read, so such calls run on the forms that read a whole pass before they write.
+bool shifted(const uint64_t *in, const uint64_t *out, size_t words) {
+  return in != out && in < out + words && out < in + words;
+}
 }  // namespace
 
 namespace cfft_internal {
@@ -135,13 +141,10 @@ int external_product_with_scratch(cfft_plan plan, const void *key_fourier, int k
   hipStream_t s = stream;
   const cfft_launch::dc64 *blk = split_w_block(plan);
   const size_t glwe_words = (size_t)k1 * 2 * plan->n;  // one GLWE: k1 polynomials of N words
-  // One launch, no scratch.  It writes a GLWE's result while later GLWEs are
-  // still to be read, so buffers that overlap other than exactly keep the
-  // split form, which reads a whole pass before it writes.
-  const size_t span = batch * glwe_words;
-  const bool shifted = glwe && out && glwe != out && glwe < out + span && out < glwe + span;
+  // one launch, no scratch
+  const bool overlap = glwe && out && shifted(glwe, out, batch * glwe_words);
   int cus = 0;
-  if (blk && !shifted && (plan->n < 2048 || plan->twist_mirrored)) {
+  if (blk && !overlap && (plan->n < 2048 || plan->twist_mirrored)) {
     e = cfft_launch::cu_count(&cus);
     if (e != hipSuccess) return hip_error(e, "external product");
   }
@@ -205,7 +208,8 @@ int cfft_exact_polymul_u64(cfft_plan plan, const uint64_t *a, const uint64_t *b,
   const cfft_launch::dc64 *blk = plan->n == 1024 ? plan->d_tw_r16
                                  : plan->n < 1024 && plan->base_n == plan->n ? plan->d_tw_base1024
                                                                              : nullptr;
-  if (blk)
+  const size_t words = batch * 2 * plan->n;
+  if (blk && !shifted(a, c, words) && !shifted(b, c, words))
     return hip_error(cfft_launch::exact_polymul_wave(ilog2(plan->n), a, b, c, margin, batch, blk,
                                                      plan->d_twist, s),
                      "exact product");

@@ -262,7 +262,9 @@ int cfft_negacyclic_polymul_u64(cfft_plan plan, const uint64_t *a, const int64_t
  * inspect the margins (that would synchronise the stream): a caller that
  * needs the guarantee passes `margin` and checks it; for 4 <= N <= 4096 it
  * stays far below 0.5 (measured 0.0098 at N = 4096 with every limb at
- * -2^15, the largest |D_3|). */
+ * -2^15, the largest |D_3|).  c may be a or b, or overlap them in any other
+ * way (every operand is then read before the first result is written, through
+ * a device scratch). */
 int cfft_exact_polymul_u64(cfft_plan plan, const uint64_t *a, const uint64_t *b, uint64_t *c,
                            double *margin, size_t batch, cfft_stream_t stream);
 /* The same exact product over the double-double transform of an fft128 plan

@@ -183,3 +183,30 @@ def test_exact_wave_groups(cfft, oracle, N, batch):
     for i in range(0, batch, 500):
         part = products.exact_polymul_u64_host(plan, a[i:i + 1], b[i:i + 1])
         assert np.array_equal(part[0], c[i]), i
+
+
+@pytest.mark.parametrize("N,base_n", [(512, 256), (1024, 512), (2048, 1024), (4096, 1024)])
+@pytest.mark.parametrize("over", ["a", "b"])
+@pytest.mark.parametrize("shift", [-1, 0, 1])
+def test_exact_result_over_an_operand(cfft, oracle, N, base_n, over, shift):
+    """c in the place of an operand, or overlapping it shifted by one product
+    in either direction: the words of separate buffers (600 products: more
+    than one round of the fused kernel at N = 2048)."""
+    from cfft_amd import check, lib
+    from cfft_amd.device import DeviceBuffer
+    from cfft_amd.unordered import FftAlgo, Method, Plan
+    print("exact over an operand: N=%d %s shift=%d" % (N, over, shift), flush=True)
+    batch = 600
+    rng = np.random.default_rng(N + shift)
+    x = rng.integers(0, M, (batch, N), dtype=np.uint64)
+    y = rng.integers(0, M, (batch, N), dtype=np.uint64)
+    plan = Plan(N // 2, Method.UserProvided(FftAlgo.Dif16, base_n))
+    pad = np.zeros((1, N), np.uint64)
+    d, other = DeviceBuffer.from_host(np.concatenate([pad, x, pad])), DeviceBuffer.from_host(y)
+    at = d.dptr + N * 8
+    ops = (at, other.dptr) if over == "a" else (other.dptr, at)
+    check(lib.cfft_exact_polymul_u64(plan.handle, *ops, at + shift * N * 8, None, batch, None))
+    got = d.download()[1 + shift:1 + shift + batch]
+    for i in list(range(0, batch, 97)) + [batch - 1]:
+        want = oracle.schoolbook_u64(x[i:i + 1], y[i:i + 1])[0]
+        assert np.array_equal(got[i], want), (i, int(np.sum(got[i] != want)))
