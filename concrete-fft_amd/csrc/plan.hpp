@@ -76,13 +76,14 @@ size_t external_product_scratch_bytes(const cfft_plan_s *plan, int k1, int level
 // and nothing is allocated (CFFT_ERROR_SIZE if one GLWE does not fit).
 // glwe_tab / out_tab (optional, device-readable, one u64 address per GLWE of
 // the batch) replace the contiguous glwe / out; they need a plan for which
-// external_product_tables_supported holds.
+// external_product_tables_supported holds.  tab_overlap: an output of the tables
+// overlaps another GLWE's input (each pass is read before it is written then).
 int external_product_with_scratch(cfft_plan_s *plan, const void *key_fourier, int k1, int levels,
                                   int base_log, const uint64_t *glwe, uint64_t *out,
                                   size_t batch, hipStream_t stream, void *scratch,
                                   size_t scratch_bytes, bool no_alloc,
                                   const uint64_t *glwe_tab = nullptr,
-                                  const uint64_t *out_tab = nullptr);
+                                  const uint64_t *out_tab = nullptr, bool tab_overlap = false);
 // the plan runs the wave-local split kernels (Dif16, n = 512, 1024, 2048),
 // which read and write GLWEs through address tables
 bool external_product_tables_supported(const cfft_plan_s *plan);

@@ -110,7 +110,7 @@ int external_product_with_scratch(cfft_plan plan, const void *key_fourier, int k
                                   int base_log, const uint64_t *glwe, uint64_t *out,
                                   size_t batch, hipStream_t stream, void *scratch,
                                   size_t scratch_bytes, bool no_alloc, const uint64_t *glwe_tab,
-                                  const uint64_t *out_tab) {
+                                  const uint64_t *out_tab, bool tab_overlap) {
   int st = check_extprod_plan(plan);
   if (st != CFFT_SUCCESS) return st;
   if (k1 < 1 || k1 > kMaxK1 || levels < 1)
@@ -142,7 +142,8 @@ int external_product_with_scratch(cfft_plan plan, const void *key_fourier, int k
   const cfft_launch::dc64 *blk = split_w_block(plan);
   const size_t glwe_words = (size_t)k1 * 2 * plan->n;  // one GLWE: k1 polynomials of N words
   // one launch, no scratch
-  const bool overlap = glwe && out && shifted(glwe, out, batch * glwe_words);
+  const bool overlap =
+      glwe && out ? shifted(glwe, out, batch * glwe_words) : tab_overlap;
   int cus = 0;
   if (blk && !overlap && (plan->n < 2048 || plan->twist_mirrored)) {
     e = cfft_launch::cu_count(&cus);

@@ -40,6 +40,7 @@
 #include "cfft.h"
 #include "launch.hpp"
 #include "plan.hpp"
+#include "serve_overlap.hpp"
 
 using cfft_internal::hip_error;
 using cfft_internal::set_error;
@@ -309,6 +310,17 @@ hipError_t cfft_server_s::launch(Batch &b) {
   int rc;
   if (b.kind == CFFT_REQUEST_EXTERNAL_PRODUCT) {
     const Key &k = keys[b.key];
+    // requests that write over each other's inputs (a chain submitted without
+    // waiting for its links) see each buffer as it was before the batch
+    bool overlap = false;
+    if (b.dev && direct && m > 1) {
+      std::vector<uint64_t> in(m), out(m);
+      for (size_t i = 0; i < m; ++i) {
+        in[i] = (uint64_t)(uintptr_t)b.reqs[i].in0;
+        out[i] = (uint64_t)(uintptr_t)b.reqs[i].out;
+      }
+      overlap = cfft_internal::outputs_meet_other_inputs(in, out, in_row_bytes);
+    }
     // the split form's Fourier scratch sits in this batch's pool block, after
     // its outputs: no allocation and no shared buffer on the serving path
     const size_t io = round_up(b.in_bytes) + round_up(m * b.reqs[0].out_bytes);
@@ -316,7 +328,7 @@ hipError_t cfft_server_s::launch(Batch &b) {
         k.plan, k.d_fourier, k.k1, k.levels, k.base_log,
         direct ? nullptr : reinterpret_cast<const uint64_t *>(d_in),
         direct ? nullptr : reinterpret_cast<uint64_t *>(d_out), m, st, d_in + io, b.dev_len - io,
-        false, direct ? tab_dev : nullptr, direct ? tab_dev + m : nullptr);
+        false, direct ? tab_dev : nullptr, direct ? tab_dev + m : nullptr, overlap);
   } else {
     cfft_plan p = plans[b.log2N].load(std::memory_order_acquire);
     rc = cfft_negacyclic_polymul_u64(p, reinterpret_cast<const uint64_t *>(d_in),

@@ -393,8 +393,12 @@ typedef enum { CFFT_REQUEST_POLYMUL = 0, CFFT_REQUEST_EXTERNAL_PRODUCT = 1 } cff
  * chain of requests on one device accumulator (a CMux chain of blind
  * rotation) stays on the device.  The inputs must be complete when the
  * request is submitted (the server does not wait on the caller's streams);
- * the output is complete when the ticket is done.  Device requests batch
- * with device requests of the same kind, N and key, up to 32767 a batch. */
+ * the output is complete when the ticket is done.  out may be the request's
+ * own input.  Over another outstanding request's input it is defined only on a
+ * server of one stream, where that request sees the whole buffer as it was
+ * before or after (a batch's inputs are read before its outputs are written).
+ * Device requests batch with device requests of the same kind, N and key, up to
+ * 32767 a batch. */
 #define CFFT_REQUEST_DEVICE_BUFFERS 0x100
 /* Host buffers (or device buffers, with CFFT_REQUEST_DEVICE_BUFFERS), owned
  * by the caller and valid until the request completes.

@@ -368,3 +368,33 @@ def test_large_host_batches(cfft):
         alone = srv.wait(srv.submit(q, keep))
         assert np.array_equal(made[i][1][-1], alone), i
     srv.close()
+
+
+@pytest.mark.parametrize("N", [1024, 2048, 4096])
+def test_device_requests_over_each_others_inputs(cfft, N):
+    """Device requests submitted together on one stream, each writing over the
+    next one's input: a request sees that buffer whole, as it was before the
+    request that writes it or after it, whichever batch it lands in."""
+    from cfft_amd.device import DeviceBuffer
+    from cfft_amd.serve import Server
+    rng = np.random.default_rng(N + 3)
+    srv = Server(streams=1)
+    keys = _setup(srv, rng, sizes=(N,))
+    kid = keys[N][0]
+    m = 400
+    data = rng.integers(0, M, (m + 1, K1, N), dtype=np.uint64)
+    bufs = [DeviceBuffer.from_host(x) for x in data]
+    tickets = [srv.submit(*srv.extprod_request_device(kid, bufs[i], bufs[i + 1]))
+               for i in range(m)]
+    for t in tickets:
+        srv.wait(t)
+    last = [b.download() for b in bufs]
+
+    def product(x):
+        out = DeviceBuffer((K1, N), np.uint64)
+        return srv.wait(srv.submit(*srv.extprod_request_device(kid, DeviceBuffer.from_host(x),
+                                                               out))).download()
+    for i in range(m):
+        assert np.array_equal(last[i + 1], product(data[i])) or \
+            np.array_equal(last[i + 1], product(last[i])), i
+    srv.close()
