@@ -27,7 +27,7 @@ class Plan:
         bufs = (re0, re1, im0, im1)
         if all(isinstance(x, DeviceBuffer) for x in bufs):
             if batch is None:
-                batch = math.prod(re0.shape) // n
+                batch = math.prod(map(int, re0.shape)) // n  # (as in ordered.py)
             f = lib.cfft128_fwd if fwd else lib.cfft128_inv
             check(f(self.handle, re0.dptr, re1.dptr, im0.dptr, im1.dptr, batch,
                     stream.handle if stream else None))

@@ -71,7 +71,7 @@ class _PlanBase:
         if not n:
             n = self._n = self.fft_size()
         if isinstance(buf, DeviceBuffer):
-            total = math.prod(buf.shape)
+            total = math.prod(map(int, buf.shape))  # (a numpy int of 32 bits would wrap)
             if buf.dtype != np.complex128:
                 raise TypeError("device buffer must be complex128")
             if batch is None:
