@@ -6,8 +6,8 @@
 // base passes of a chunk stay within one wavefront and exchange through LDS
 // without a workgroup barrier; depth passes run over the whole transform.  A
 // pass takes its butterflies' inputs from registers (first pass) or LDS,
-// requests the next pass's twiddles as soon as it has used its own, so that
-// they arrive during the exchange, and leaves its outputs in LDS or (last
+// requests the next pass's twiddles as soon as it has used its own (or has stored
+// its outputs, passes8), so that they arrive during the exchange, and leaves its outputs in LDS or (last
 // pass) in registers.  Every thread's inputs and outputs of a whole transform
 // are the same eight points, so loads, twist, pointwise product and the
 // hand-over from a forward to an inverse transform need no exchange.
@@ -187,8 +187,10 @@ __device__ __forceinline__ void bf16_pair(c64 *v, uint32_t o) {
 // passes PI ... of F: v[m] holds the thread's point m on entry of the first
 // pass (slot order of `linear8`) and on exit of the last; w holds pass PI's
 // twiddles.  `x`: n + n / 16 points of LDS; the caller's earlier reads of it
-// by other threads must be complete.
-template <class F, int PI>
+// by other threads must be complete.  LATE: the next pass's twiddles are
+// requested once its points are in LDS and no longer in registers (for callers
+// that hold another transform meanwhile), else before those are stored.
+template <class F, int PI, bool LATE = false>
 __device__ __forceinline__ void passes8(c64 *v, c64 *w, c64 *x, const Lane8<F> &L0,
                                         const c64 *__restrict__ tw) {
   using Q = Pass8<F, PI>;
@@ -245,7 +247,7 @@ __device__ __forceinline__ void passes8(c64 *v, c64 *w, c64 *x, const Lane8<F> &
       for (int k = 0; k < 8 / Q::NB; ++k) v[i + k * Q::NB] = y[i * (8 / Q::NB) + k];
   } else {
     c64 wn[8];
-    twiddles8<F, PI + 1>(L, pass_opaque(tw), wn);
+    if constexpr (!LATE) twiddles8<F, PI + 1>(L, pass_opaque(tw), wn);
     // every reader of the exchange's previous contents is done
     if constexpr (!first) {
       if constexpr (wave_in) wave_lds_fence();
@@ -260,10 +262,14 @@ __device__ __forceinline__ void passes8(c64 *v, c64 *w, c64 *x, const Lane8<F> &
         x[lds_pad(out_point<F, Q>(base, bb, Q::p16 ? pair_out(L, k) : (uint32_t)k))] =
             y[i * (8 / Q::NB) + k];
     }
+    if constexpr (LATE) {
+      sched_fence();
+      twiddles8<F, PI + 1>(Lane8<F>(launder_u32(L0.lt)), pass_opaque(tw), wn);
+    }
     constexpr bool wave_out = !Q::depth && !Pass8<F, PI + 1>::depth && F::TC <= 64;
     if constexpr (wave_out) wave_lds_fence();
     else __syncthreads();
-    passes8<F, PI + 1>(v, wn, x, L0, tw);
+    passes8<F, PI + 1, LATE>(v, wn, x, L0, tw);
   }
 }
 

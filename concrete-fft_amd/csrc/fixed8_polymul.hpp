@@ -2,8 +2,9 @@
 // eight-point schedule.
 //
 // What bounds it: latency and LDS exchanges, at 16 waves per CU (eight points
-// of a transform are 32 registers, so a product's two operands stay under 128
-// and four waves run per SIMD).  Against the same programs with an exchange
+// of a transform are 32 registers; a product's two operands are held to 128, so
+// that four waves run per SIMD: up to n = 1024 and for Dif16 some instances spill
+// 12 to 28 bytes per lane for it).  Against the same programs with an exchange
 // through LDS around every pass and transform, twiddles gathered from the
 // n-point table after each butterfly (k_polymul_fixed, us): N = 2048 Dif4 / 512
 // 14.6 -> 9.2 (1 product), 25.1 -> 18.7 (1024), 147.8 -> 121 (8192); Dit8 / 512
@@ -43,6 +44,13 @@ k_polymul_fixed8(const uint64_t *__restrict__ A, const int64_t *__restrict__ B,
   using F = Fixed8<ALGO, LOG2N, LOG2BN, true>;
   using I = Fixed8<ALGO, LOG2N, LOG2BN, false>;
   using Ge = Geom8<LOG2N>;
+  // From n = 2048 on a pass's twiddles wait for its points to leave the registers:
+  // requested before that, 27 of the 41 instances spilled 12-44 bytes per lane (now
+  // Dif16's, 12-20, which measured the same either way).  us, so and now: N = 16384
+  // Dif4 / 1024 42.5 / 37.4 (1 product), 196 / 174 (1024), Dit4 / 1024 40.8 / 36.6,
+  // 189 / 171; N = 8192 Dif8 / 1024 93 / 85 (1100), Dif4 / 1024 98 / 95; N = 4096
+  // Dif8 / 512 39.2 / 37.5.  Up to n = 1024 it made no difference (0.98-1.03x).
+  constexpr bool LATE = LOG2N >= 11 && !F::pair;
   constexpr uint32_t n = F::n;
   constexpr int LI = (int)I::prog.npass - 1;
   extern __shared__ c64 smem[];
@@ -81,7 +89,7 @@ k_polymul_fixed8(const uint64_t *__restrict__ A, const int64_t *__restrict__ B,
     rb[2 * m + 1] = ld_stream(&b[j + n]);
   }
   sched_fence();
-  passes8<F, 0>(fa, w, x, L, tw);
+  passes8<F, 0, LATE>(fa, w, x, L, tw);
   {
     const Lane8<F> L1(launder_u32(lt));
     const c64 *tz = launder(twist);
@@ -91,13 +99,13 @@ k_polymul_fixed8(const uint64_t *__restrict__ A, const int64_t *__restrict__ B,
       fb[m] = cmul(tz[linear8<F, 0>(L1, m)], mk(i64_to_f64(rb[2 * m]), i64_to_f64(rb[2 * m + 1])));
   }
   settled();
-  passes8<F, 0>(fb, w, x, L, tw);
+  passes8<F, 0, LATE>(fb, w, x, L, tw);
 #pragma unroll
   for (int m = 0; m < 8; ++m) fa[m] = cmul(fa[m], fb[m]);
   const Lane8<I> Li(launder_u32(lt));
   twiddles8<I, 0>(Li, launder(tw), w);
   settled();
-  passes8<I, 0>(fa, w, x, Li, tw);
+  passes8<I, 0, LATE>(fa, w, x, Li, tw);
   if (poly >= batch) return;
   const c64 *uz = launder(untwist);
   const Lane8<I> Lo(launder_u32(lt));

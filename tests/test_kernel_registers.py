@@ -38,3 +38,18 @@ def test_one_launch_external_product_keeps_its_registers():
     spilled = {k[".name"]: k[".private_segment_fixed_size"] for k in fused
                if k[".private_segment_fixed_size"]}
     assert not spilled, spilled
+
+
+def test_eight_point_products_keep_their_registers():
+    """n = 2048 ... 8192, every algo but Dif16 (whose radix-16 lane pairs keep
+    12 to 20 bytes)."""
+    from cfft_amd._lib import LIB_PATH
+    found, spilled = 0, {}
+    for k in kernels(LIB_PATH):
+        m = re.search(r"k_polymul_fixed8ILi(\d+)ELi(\d+)E", k[".name"])
+        if not m or int(m.group(1)) == 6 or int(m.group(2)) < 11:
+            continue
+        found += 1
+        if k[".private_segment_fixed_size"]:
+            spilled[k[".name"]] = k[".private_segment_fixed_size"]
+    assert found == 36 and not spilled, (found, spilled)
