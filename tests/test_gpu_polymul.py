@@ -265,16 +265,20 @@ def test_dif16_product_routes_meet(cfft, oracle, N, base_n):
 
 @pytest.mark.parametrize("N,batch", [(4096, 513), (4096, 1024), (4096, 1281), (8192, 257),
                                      (8192, 511), (8192, 770), (16384, 129), (16384, 259)])
-def test_depth_product_rounds(cfft, oracle, N, batch):
+def test_depth_product_partial_rounds(cfft, oracle, N, batch):
     """Register-resident products with a depth pass: batches that end inside
-    a round, one group of a workgroup after another; every product equals the
-    eight-point kernel's (small batches) and the oracle's at both ends."""
+    a round, one group of a workgroup after another.  At N = 4096 and 8192 every
+    product equals the eight-point kernel's (which small batches run on) and the
+    oracle's at both ends; at N = 16384, where every batch runs on the kernel
+    with the depth pass, every product equals the oracle's."""
     from cfft_amd import products
     from cfft_amd.unordered import FftAlgo, Method, Plan
     print("N=%d batch=%d" % (N, batch), flush=True)
     plan = Plan(N // 2, Method.UserProvided(FftAlgo.Dif16, 1024))
     a, b = rand_inputs(N + batch, batch, N)
     got = products.negacyclic_polymul_u64_host(plan, a, b)
+    if N == 16384:
+        assert np.array_equal(got, oracle.polymul_f64(a, b, 6, 1024, threads=16))
     for i in range(0, batch, 128):
         assert np.array_equal(products.negacyclic_polymul_u64_host(
             plan, a[i:i + 128], b[i:i + 128]), got[i:i + 128]), i
