@@ -106,11 +106,13 @@ def test_external_product_errors(cfft):
                                   o, 1)
 
 
+@pytest.mark.parametrize("k1", [2, 5])
 @pytest.mark.parametrize("N", [1024, 2048, 4096])
-def test_batch_splits_agree(cfft, oracle, N):
-    # one call over 200 GLWEs equals two calls over 100 each (different
-    # launch shapes of the split row / column kernels) and the oracle
-    k1, levels, base_log = 2, 3, 8
+def test_batch_splits_agree(cfft, oracle, N, k1):
+    # one call over 200 GLWEs equals two calls over 100 each and the oracle
+    # (different launch shapes: GLWEs per workgroup of the one-launch form at
+    # k1 = 2, the split form's row and column kernels at k1 = 5)
+    levels, base_log = 3, 8
     rng = np.random.default_rng(N + 99)
     key = rng.integers(0, M, (k1 * levels, k1, N), dtype=np.uint64)
     glwe = rng.integers(0, M, (200, k1, N), dtype=np.uint64)
@@ -126,23 +128,30 @@ def test_batch_splits_agree(cfft, oracle, N):
                                                                 min(N // 2, 1024), glwe[b]))
 
 
-def test_large_batch_runs_in_passes(cfft, oracle):
-    # k1 * levels = 16 rows per GLWE: 16384 rows make one pass of 1024 GLWEs,
-    # so 1100 GLWEs run in two passes over the same scratch
-    N, k1, levels, base_log = 1024, 2, 8, 4
+@pytest.mark.parametrize("k1,levels,algo,base_n", [
+    (2, 8, 6, 512),   # the one-launch form: no passes
+    (1, 16, 6, 512),  # wave-local split kernels, 16 rows per GLWE
+    (5, 4, 6, 512),   # ... 20 rows: passes of 819 GLWEs
+    (2, 8, 2, 512),   # generic split kernels (Dif4 plan), 16 rows
+])
+def test_large_batch_runs_in_passes(cfft, oracle, k1, levels, algo, base_n):
+    # the split form takes 16384 rows in a pass: with 16 rows per GLWE 1100 GLWEs
+    # run in two passes (of 1024 and 76) over the same scratch
+    N, base_log = 1024, 4
     rng = np.random.default_rng(321)
     key = rng.integers(0, M, (k1 * levels, k1, N), dtype=np.uint64)
     glwe = rng.integers(0, M, (1100, k1, N), dtype=np.uint64)
-    plan = _plan(N, 6, 512)
+    plan = _plan(N, algo, base_n)
     kf = _key_fourier(plan, key, k1, levels)
     whole = _extprod(plan, kf, k1, levels, base_log, glwe)
     parts = np.concatenate([_extprod(plan, kf, k1, levels, base_log, glwe[i:j])
                             for i, j in ((0, 500), (500, 1100))])
     assert np.array_equal(whole, parts)
-    kfh = oracle.torus_to_fourier(key, 6, 512)
-    for b in (0, 1023, 1024, 1099):
-        assert np.array_equal(whole[b], oracle.external_product(N, k1, levels, base_log, kfh, 6,
-                                                                512, glwe[b])), b
+    kfh = oracle.torus_to_fourier(key, algo, base_n)
+    per_pass = 16384 // (k1 * levels)
+    for b in (0, per_pass - 1, per_pass, 1099):
+        assert np.array_equal(whole[b], oracle.external_product(N, k1, levels, base_log, kfh,
+                                                                algo, base_n, glwe[b])), b
 
 
 @pytest.mark.parametrize("N,k1,levels,base_log,batch", [
