@@ -156,15 +156,18 @@ __global__ void __launch_bounds__(512) k_exact_inv(const c64 *__restrict__ F,
 // weights are added, and the rounding distance is only formed when the caller
 // asks for the margin.
 //
-// What bounds it: a round (two products of N = 2048, 24 transforms) takes 19.5
-// us, of which LDS traffic is about 9 and VALU issue about 10; the barriers
-// keep the waves in the same phase, so they add up.  Two 4-wave workgroups per
-// CU (twist from global memory) took 81.0 us for 2048 products against 78.4;
-// requesting the next round's words during the inverse or the sums 79-81.
-// Before (us): N = 2048, 2048 products 88 -> 78.4, 64 products 22.1 -> 14.5, one
-// 16.1 -> 13.7 (one workgroup per two products, tables staged by each, generic
-// limbs); on the two-kernel form N = 1024, 4096 products 373 -> 75, one 40 ->
-// 13; N = 512, 8192 products 319 -> 72.
+// What bounds it: a round (two products of N = 2048, 24 transforms) takes 19.5-20
+// us; by the counters (N = 2048 x 2048) the SIMDs issue VALU instructions for 52 %
+// of it and LDS is busy for 30 %, and a wave waits for data or barriers 31 % and
+// to issue 34 % of its time: the barriers keep the two waves of a SIMD in the same
+// phase, so the phases add up.  Two 4-wave workgroups per CU (twist from global
+// memory) took 81.0 us for 2048 products against 78.4; requesting the next round's
+// words during the inverse or the sums 79-81.
+// Before (us): N = 2048, 2048 products 87.5-88.5 -> 78.8-81.5 over three devices, 40
+// products 22.2 -> 14.7, one 16.2 -> 13.7 (one workgroup per two products, tables
+// staged by each, generic limbs); on the two-kernel form N = 1024, 4096 products
+// 373 -> 75, one 40 -> 13; N = 512, 8192 products 320 -> 69.  (The forms for N = 512
+// and 1024 that also return the margin spill 12 bytes per lane.)
 constexpr uint32_t kXW = 8;
 constexpr uint32_t kXTw = 16 * 64 + 16 * 4;
 constexpr size_t kXLds = (kXTw + kXW * R16<10>::lds_words) * sizeof(c64);

@@ -115,6 +115,7 @@ __host__ __device__ __forceinline__ uint32_t pad128(uint32_t i) { return i + (i 
 // costs (us: n = 1024 x 1000 inverse 45.2 -> 37.8, n = 512 x 4096 forward 89.5 ->
 // 65.6, n = 64 x 32768 forward 80.4 -> 56.7).
 constexpr uint32_t kRB = 2;
+static_assert(kRB == 2, "a round that is not full has one stage");
 __host__ __device__ __forceinline__ uint32_t fft128_blocks_per_wg(uint32_t L) {
   return L >= 6 + kRB ? 1u : 1u << (6 + kRB - L);
 }
@@ -290,8 +291,6 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))
     const uint32_t ptop = lo_bit + nb - 1;
     if (nb == kRB)
       run_round<(int)kRB, FWD, MULV>(lds, g, first, last, ptop, L, Lg, jhi, lt, T, tw, active);
-    else if (kRB == 3 && nb == 2)
-      run_round<2, FWD, MULV>(lds, g, first, last, ptop, L, Lg, jhi, lt, T, tw, active);
     else
       run_round<1, FWD, MULV>(lds, g, first, last, ptop, L, Lg, jhi, lt, T, tw, active);
   }

@@ -55,7 +55,8 @@ int cfft_external_product_noalloc(cfft_plan plan, const void *key_fourier, int k
   const int rc = device_scratch(&s);
   if (rc != CFFT_SUCCESS) return rc;
   // the split kernels write every spectrum of a pass before reading it, so
-  // the scratch needs no clearing between calls
+  // the scratch needs no clearing between calls (the one-launch form, which
+  // takes k1 = 2 ... 4 on Dif16 plans, uses none of it)
   return cfft_internal::external_product_with_scratch(plan, key_fourier, k1, levels, base_log,
                                                       glwe, out, batch, (hipStream_t)stream, s,
                                                       kScratchBytes, true);

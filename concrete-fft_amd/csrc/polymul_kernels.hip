@@ -340,10 +340,13 @@ __device__ __forceinline__ void depth_raw_to_lds(const DepthRaw<LOG2N> &d, c64 *
 // batch below G per CU) is spread over the CUs, one product on each, where
 // two or four of them on part of the CUs had left the others idle (N = 4096:
 // 600 products 26.4 -> 23.3 us, 1100 47.2 -> 39.3; N = 8192: 600 48.8 -> 43.3;
-// batches that fill every round the same within 1 %).  A group whose share is
-// done ends; a barrier waits on the waves that are left.  A barrier of each
-// product's own (a counter in LDS) instead of the workgroup's was slower:
-// 33.3 against 30.1 us for 512 products of N = 8192.
+// 777 52.0 -> 51.3; batches that fill every round the same within 1 %).  A group is
+// whole waves (128 threads or more), and one whose share is done ends while the
+// others still meet at the workgroup's barriers: the hardware's barrier
+// (s_barrier) waits for the waves that have not ended, which __syncthreads by
+// itself does not promise.  A barrier of each product's own (a counter in LDS)
+// instead of the workgroup's was slower: 33.3 against 30.1 us for 512 products of
+// N = 8192.
 template <int LOG2N, bool PRE_B, bool PRE_A>
 __global__ void __launch_bounds__(64 * kPW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_depth_polymul(const uint64_t *__restrict__ A, const int64_t *__restrict__ B,

@@ -12,8 +12,8 @@
 //      memory -- and launches it: one host-to-device copy, one batched kernel,
 //      one device-to-host copy, one event (device-buffer requests: the
 //      callers' device buffers are named by a table of addresses in mapped
-//      pinned staging; the wave-local external-product kernels read and
-//      write them through it, other batches are gathered into the batch's
+//      pinned staging; the one-launch and wave-local external-product kernels
+//      read and write them through it, other batches are gathered into the batch's
 //      block by a kernel and scattered back by another; nothing crosses the
 //      bus but the table);
 //   3. sleeps until a submission arrives, or polls while batches are in flight.
@@ -267,7 +267,7 @@ hipError_t cfft_server_s::launch(Batch &b) {
   const size_t in_rows = b.kind == CFFT_REQUEST_EXTERNAL_PRODUCT ? m : 2 * m;
   const size_t in_row_bytes = b.kind == CFFT_REQUEST_EXTERNAL_PRODUCT ? b.reqs[0].in_bytes : N * 8;
   hipError_t e = hipSuccess;
-  // external products on the wave-local split kernels read and write
+  // external products on Dif16 plans of N = 1024 ... 4096 read and write
   // through an address table: the callers' device buffers, or for a small
   // host-buffer batch the request slots of the mapped pinned staging
   const bool tables = b.kind == CFFT_REQUEST_EXTERNAL_PRODUCT &&
@@ -322,7 +322,9 @@ hipError_t cfft_server_s::launch(Batch &b) {
       overlap = cfft_internal::outputs_meet_other_inputs(in, out, in_row_bytes);
     }
     // the split form's Fourier scratch sits in this batch's pool block, after
-    // its outputs: no allocation and no shared buffer on the serving path
+    // its outputs: no allocation and no shared buffer on the serving path (it is
+    // reserved for every batch, though most run on the one-launch form: which
+    // form a batch takes depends on its size and on `overlap`)
     const size_t io = round_up(b.in_bytes) + round_up(m * b.reqs[0].out_bytes);
     rc = cfft_internal::external_product_with_scratch(
         k.plan, k.d_fourier, k.k1, k.levels, k.base_log,
