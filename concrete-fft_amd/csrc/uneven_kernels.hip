@@ -468,7 +468,7 @@ __device__ __forceinline__ void leave_queue(uint32_t *ctr, uint32_t nw) {
 // index when a tile starts and publishes it when the tile ends, so the
 // atomic's round trip overlaps the tile.  (Clearing the counters by a launch
 // of their own costs 1.2-1.9 us: 1 job 9.6 -> 11.6, 50 28.4 -> 30.1, 1000 31.7 ->
-// 33.2, 3000 60.6 -> 61.9; at 20 000, 377 us, it is within what boxes differ by.)
+// 33.2, 3000 60.6 -> 61.9; at 20 000, 377 us, it is within what devices differ by.)
 // Without `counter` the tiles are dealt round-robin (workgroup w: tiles w,
 // w + G, ...).  Device-scope atomics on one address are serialised (measured
 // ~50 ns each); the partitions divide that cost, the static deal removes it.

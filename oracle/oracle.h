@@ -4,7 +4,7 @@
  *
  * TEST INFRASTRUCTURE ONLY.  Nothing in the shipped library includes, links or
  * calls this code: only tests/, __graft_entry__.smoke() and bench.py's
- * cpu_baseline leg load liboracle.so, and only as the checker (or as the
+ * cpu_baseline leg load liboracle.so, and only as the oracle (or as the
  * timed CPU comparison).  Every function cites the reference file:line whose
  * arithmetic it restates.
  *

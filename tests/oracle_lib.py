@@ -1,4 +1,4 @@
-"""ctypes loader of oracle/liboracle.so (the CPU restatement used as checker).
+"""ctypes loader of oracle/liboracle.so (the CPU restatement that is the oracle).
 
 Test infrastructure: only tests, __graft_entry__.smoke() and bench.py's
 cpu_baseline leg use this module.
